@@ -29,11 +29,16 @@ INF_DEPTH = 0x3F3F3F3F
 _lib: Optional[ctypes.CDLL] = None
 
 
+def have_reference() -> bool:
+    """The reference's CPU programs can be built: their sources are there (the folder may be empty)."""
+    return os.path.isdir(os.path.join(REFERENCE_ROOT, "evaluation"))
+
+
 def build(force: bool = False, ref: bool = True) -> None:
     """Compile the oracle (and the reference CPU programs when the sources exist)."""
     if force or not os.path.exists(LIB_PATH):
         subprocess.run(["make", "-s", "-C", HERE, "-B" if force else "all"], check=True)
-    if ref and os.path.isdir(REFERENCE_ROOT):
+    if ref and have_reference():
         subprocess.run(["make", "-s", "-C", HERE, "ref", f"REF={REFERENCE_ROOT}"], check=True)
 
 
