@@ -418,6 +418,15 @@ __device__ __forceinline__ void vst(T* p, T v) {
     *(volatile __attribute__((address_space(3))) T*)(p) = v;
 }
 
+// A pointer known to address LDS (never pass one that may not), for plain ds_ accesses to a
+// wave's scratch between wave_sync()s.
+template <typename T>
+using lds_array = __attribute__((address_space(3))) T*;
+template <typename T>
+__device__ __forceinline__ lds_array<T> lds(T* p) {
+    return (lds_array<T>)(p);
+}
+
 __device__ __forceinline__ uint64_t now_ticks() { return wall_clock64(); }
 
 // Serve mode. The host's control words sit in pinned host memory; a system-scope read of

@@ -56,6 +56,32 @@ struct HasWaveQueue<P, decltype((void)P::kWaveQueue)> {
     static constexpr int value = P::kWaveQueue;
 };
 
+// A program may finish its lane tasks' bodies on the whole wave (P::run_coop): a task whose
+// run() sets lane.coop and finishes leaves the rest of its body to run_coop, which all 64
+// lanes enter once per round, after every lane's run(), with the mask of the tasks that asked.
+// Lanes without a task, and lanes whose task is short, then share the long ones' work.
+template <class P, class = void>
+struct HasCoop {
+    static constexpr bool value = false;
+};
+template <class P>
+struct HasCoop<P, decltype((void)P::kCoop)> {
+    static constexpr bool value = P::kCoop;
+};
+
+// Most tasks a batch holds: 64, or what the program asks for with its launch arguments
+// (P::batch_cap(args), 1..64). With long task bodies that the whole wave shares (run_coop), a
+// batch of c tasks takes c / 64 of the time of a full one, and the tasks it leaves are
+// published for idle waves.
+template <class P, class = void>
+struct BatchCap {
+    __device__ __forceinline__ static uint32_t of(const typename P::Args&) { return (uint32_t)kWave; }
+};
+template <class P>
+struct BatchCap<P, decltype((void)&P::batch_cap)> {
+    __device__ __forceinline__ static uint32_t of(const typename P::Args& a) { return P::batch_cap(a); }
+};
+
 // Per-wave scheduler state in LDS.
 //
 // The private end of each queue (positions [bottom, tail)) is mirrored in a ring of 64
@@ -731,6 +757,7 @@ struct Lane {
     uint32_t outcome;
     bool lds;               // the record's header and first FW frame words are not in HBM yet
     bool sum_join;          // the pending taskwait is an additive join
+    bool coop;              // run_coop finishes this task's body (HasCoop programs)
     int64_t jsum;           // sum of the children's results, after an additive join
     uint64_t join_delta;    // what finishing adds to the parent's join word
     uint32_t frame[FW];     // the first frame words, loaded when the round starts
@@ -1244,7 +1271,7 @@ __device__ __forceinline__ uint32_t pick_victim(const GtapDev& dev, uint32_t me,
 template <class P>
 __device__ __forceinline__ uint32_t try_steal_any(const GtapDev& dev, uint32_t me, uint32_t cq, uint32_t& rng,
                                                   uint32_t& tid_out, bool& idle_registered, LoopStats& st,
-                                                  uint32_t& q_out) {
+                                                  uint32_t& q_out, uint32_t max_items) {
     constexpr uint32_t Q = (uint32_t)P::kQueues;
     const int lane = lane_id();
     if (dev.nworkers < 2) return 0;
@@ -1268,7 +1295,8 @@ __device__ __forceinline__ uint32_t try_steal_any(const GtapDev& dev, uint32_t m
     sz = shfl(sz, src);
     q = uniform(shfl(q, src));
     uint32_t k = (uint32_t)(sz + 1) / 2;
-    const uint32_t batch_cap = ((int)q == HasWaveQueue<P>::value) ? 1u : dev.steal_batch;
+    uint32_t batch_cap = ((int)q == HasWaveQueue<P>::value) ? 1u : dev.steal_batch;
+    if (batch_cap > max_items) batch_cap = max_items;
     if (k > batch_cap) k = batch_cap;
     if (k == 0) k = 1;
     if (dev.term_mode == GTAP_TERM_QUIESCE && idle_registered) {
@@ -1557,6 +1585,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
     L.me = me;
     L.rs = pool_rsrc(dev.recs);
     constexpr int QL = CtxShape<P>::kQL;
+    const uint32_t bcap = BatchCap<P>::of(args);
 
     uint32_t rng = 0x9E3779B9u ^ (me * 0x85EBCA6Bu) ^ ((uint32_t)lane * 0xC2B2AE35u) ^ (uint32_t)t_begin;
     if (rng == 0) rng = 1;
@@ -1610,7 +1639,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
             for (int i = 0; i < Q && n == 0 && idle_iter == 0 && Sched != kSchedGQ; ++i) {
                 const uint32_t q = (cq + (uint32_t)i) % (uint32_t)Q;
                 if constexpr (Sched == kSchedCL) n = cl_pop_batch<P>(dev, w, me, q, my_tid);
-                else n = try_pop<P>(dev, w, me, q, my_tid);
+                else n = try_pop<P>(dev, w, me, q, my_tid, bcap);
                 if (n) {
                     vst(&w->cur_queue, q);
                     st.pops += 1;
@@ -1625,14 +1654,14 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
             if (n == 0) {
                 if constexpr (kStealAnyQueue && Sched == kSchedWS && Q > 1) {
                     uint32_t sq = 0;
-                    n = try_steal_any<P>(dev, me, cq, rng, my_tid, idle_registered, st, sq);
+                    n = try_steal_any<P>(dev, me, cq, rng, my_tid, idle_registered, st, sq, bcap);
                     if (n) batch_q = (int)sq;
                 } else {
 #pragma unroll
                     for (int i = 0; i < Q && n == 0; ++i) {
                         const uint32_t q = (cq + (uint32_t)i) % (uint32_t)Q;
                         if constexpr (Sched == kSchedGQ) n = gq_pop<P>(dev, q, my_tid, idle_registered, st);
-                        else n = try_steal<P>(dev, me, q, rng, my_tid, idle_registered, st, Sched == kSchedCL ? 1u : (uint32_t)kWave);
+                        else n = try_steal<P>(dev, me, q, rng, my_tid, idle_registered, st, Sched == kSchedCL ? 1u : bcap);
                         if (n) batch_q = (int)q;
                     }
                 }
@@ -1649,7 +1678,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
 #pragma unroll 1
                     for (int i = 0; i < Q && n == 0; ++i) {
                         const uint32_t q = (cq + (uint32_t)i) % (uint32_t)Q;
-                        const uint32_t cap = ((int)q == WQ) ? 1u : (uint32_t)kWave;
+                        const uint32_t cap = ((int)q == WQ) ? 1u : bcap;
                         const uint64_t got = ovf_pop(ovf_view(dev), q, cap, idle_registered ? 1 : 0);
                         const uint32_t code = uniform((uint32_t)got);
                         if (code & kOvfLeftIdle) idle_registered = false;
@@ -1741,6 +1770,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         uint64_t fin_delta = ~0ull;  // added to the parent's join word: -1, plus value << 16 (additive join)
         bool fin_sum = false;        // the parent waits in an additive join
         bool fin = false, sus = false;
+        if constexpr (HasCoop<P>::value) L.coop = false;
         if (WQ >= 0 && batch_q == WQ) {
             // one wave-cooperative task on all lanes
             uint32_t wt = uniform(my_tid);
@@ -1788,6 +1818,10 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                 GTAP_DEVICE_ERROR(dev, GTAP_ERROR_INVALID_FUNCTION, fin_tid, -1, fin_parent, dev.nrecs + dev.nanchors);
                 fin_parent = kNoParent;
             }
+        }
+        if constexpr (HasCoop<P>::value) {
+            const uint64_t cm = ballot(L.coop);
+            if (cm) P::run_coop(L, cm, reinterpret_cast<typename P::WaveShared*>(wave_shared));
         }
         phase_mark(PH_RUN);
 
@@ -1856,7 +1890,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                 kmax = (uint32_t)q;
             }
         }
-        const uint32_t keep_cap = ((int)kmax == WQ) ? 1u : (uint32_t)kWave;
+        const uint32_t keep_cap = ((int)kmax == WQ) ? 1u : bcap;
         uint32_t keep = cmax < keep_cap ? cmax : keep_cap;
         uint32_t next_tid = 0, next_slot = 0;
         bool next_lds = false;
@@ -1980,9 +2014,9 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         // its deque word, so the next round runs up to 64 tasks instead of waiting until the
         // wave runs dry. Their records are in HBM and load at the round's start.
         if constexpr (Sched == kSchedWS) {
-            if (keep < (uint32_t)kWave && (int)kmax != WQ) {
+            if (keep < bcap && (int)kmax != WQ) {
                 uint32_t ptid = 0;
-                const uint32_t k = try_pop<P>(dev, w, me, kmax, ptid, (uint32_t)kWave - keep);
+                const uint32_t k = try_pop<P>(dev, w, me, kmax, ptid, bcap - keep);
                 if (k) {
                     const int src = lane - (int)keep;
                     const uint32_t v = shfl(ptid, src < 0 ? 0 : src);

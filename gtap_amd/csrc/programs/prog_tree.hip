@@ -50,6 +50,7 @@ struct TreeArgs {
     const double* input;
     uint32_t input_mask;  // input_n - 1 (input_n a power of two)
     double* out;
+    uint32_t batch;  // most nodes a wave takes at once
 };
 
 __host__ __device__ __forceinline__ uint32_t xs32(uint32_t x) {
@@ -65,46 +66,36 @@ __device__ __forceinline__ uint32_t sat_u32(double v) {
     return (uint32_t)v;
 }
 
-// Memory phase: 8 loads in flight at a time, summed in order.
-__device__ __forceinline__ double node_work(const TreeArgs& g, int32_t node, int32_t mem_ops, int32_t compute_iters) {
-    const uint32_t seed = xs32((uint32_t)node ^ 0x9e3779b9u);
-    double acc = 0.0;
-    constexpr int kBatch = 8;
-    for (int32_t m0 = 0; m0 < mem_ops; m0 += kBatch) {
-        double v[kBatch];
-#pragma unroll
-        for (int j = 0; j < kBatch; ++j) {
-            const uint32_t r = xs32(seed + (uint32_t)(m0 + j) * 747796405u);
-            v[j] = (m0 + j < mem_ops) ? g.input[r & g.input_mask] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kBatch; ++j)
-            if (m0 + j < mem_ops) acc += v[j];
-    }
-    uint32_t mix = (0x9e3779b9u ^ (uint32_t)node) + sat_u32(acc);
-    for (int32_t it = 0; it < compute_iters; ++it) {
-        const double x = (double)xs32(seed + (uint32_t)it * 747796405u);
-        const double y = __builtin_fma(x, 1.0000001192092896, 0.9999999403953552);
-        mix ^= (uint32_t)__builtin_bit_cast(uint64_t, y);
-    }
-    return (double)mix;
+// One term of the arithmetic phase: the low word of fma(x, c, d). The terms are combined by
+// exclusive or, so any lane may compute any of them.
+__device__ __forceinline__ uint32_t mix_term(uint32_t seed, uint32_t it) {
+    const double x = (double)xs32(seed + it * 747796405u);
+    return (uint32_t)__builtin_bit_cast(uint64_t, __builtin_fma(x, 1.0000001192092896, 0.9999999403953552));
 }
 
 constexpr int kUnusedSlot = 16;  // frame bytes 16..23
+constexpr int kCoopReads = 4;    // reads in flight per lane of a group
 
 struct Program {
     static constexpr int kQueues = 1;
+    static constexpr bool kCoop = true;    // node work is done by run_coop
     static constexpr int kFrameWords = 4;  // node, height, mem_ops, compute_iters
     static constexpr uint32_t kMaxFunc = F_NODE;
     static constexpr uint32_t kFrameBytes = 24;
     using Args = TreeArgs;
+    struct WaveShared {
+        double v[kCoopReads * kWave];  // the input values read in one step, in read order per node
+        int32_t src[kWave];            // lanes that hold the round's nodes
+    };
+    __device__ __forceinline__ static uint32_t batch_cap(const Args& a) { return a.batch; }
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
+    template <class L>
+    __device__ __forceinline__ static void run_coop(L& lane, uint64_t mask, WaveShared* sh);
 };
 
 template <class L>
 __device__ __forceinline__ void Program::run(L& lane) {
-    const TreeArgs& g = *lane.args;
     const int32_t node = lane.template arg<int32_t>(0);
     const int32_t height = lane.template arg<int32_t>(4);
     const int32_t mem_ops = lane.template arg<int32_t>(8);
@@ -119,7 +110,7 @@ __device__ __forceinline__ void Program::run(L& lane) {
             }
             [[fallthrough]];
         case 1:
-            g.out[node] = node_work(g, node, mem_ops, iters);
+            lane.coop = true;  // the node's work: run_coop
             __gtap_finish_task(lane);
             return;
         default:
@@ -127,6 +118,57 @@ __device__ __forceinline__ void Program::run(L& lane) {
             __gtap_finish_task(lane);
             return;
     }
+}
+
+// The work of a round's m nodes on all 64 lanes. A level of the tree takes at least one node's
+// work, and on one lane that is 64 reads 8 at a time and a chain of 512 steps, about 25 us: it
+// bound the whole run (height 15, 64 reads, 512 steps: 663 us, with most waves idle). Here each
+// node gets a group of g lanes, the largest power of two <= 64 / m: the reads go through LDS and
+// every lane of the group sums them in order, so the sum has the same bits; the arithmetic terms
+// are divided among the lanes and combined by exclusive or. With full batches 368 us, with the
+// batches of at most 8 nodes that gtap_tree asks for 196 us, now bound by the rounds' own latency
+// (the same tree without node work takes 135 us).
+template <class L>
+__device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
+    const TreeArgs& a = *lane.args;
+    const int32_t l = lane_id();
+    const int32_t m = popc(mask);
+    int32_t g = kWave;
+    while (g * m > kWave) g >>= 1;
+    if (lane.coop) vst(&sh->src[rank_in(mask)], l);
+    wave_sync();
+    const int32_t grp = l / g, sub = l % g;
+    const bool on = grp < m;
+    const int32_t src = vld(&sh->src[on ? grp : 0]);
+    const int32_t node = shfl((int32_t)lane.frame[0], src);
+    int32_t mem_ops = shfl((int32_t)lane.frame[2], src);
+    int32_t iters = shfl((int32_t)lane.frame[3], src);
+    if (!on) mem_ops = iters = 0;
+    const uint32_t seed = xs32((uint32_t)node ^ 0x9e3779b9u);
+    double acc = 0.0;
+    lds_array<double> buf = lds(&sh->v[grp * g * kCoopReads]);
+    const int32_t step = g * kCoopReads;
+    for (int32_t m0 = 0; ballot(m0 < mem_ops); m0 += step) {
+        double v[kCoopReads];
+#pragma unroll
+        for (int j = 0; j < kCoopReads; ++j) {
+            const int32_t k = m0 + j * g + sub;
+            v[j] = k < mem_ops ? a.input[xs32(seed + (uint32_t)k * 747796405u) & a.input_mask] : 0.0;
+        }
+        wave_sync();  // the previous step's values have been read
+#pragma unroll
+        for (int j = 0; j < kCoopReads; ++j) buf[j * g + sub] = v[j];
+        wave_sync();
+        const int32_t cnt = mem_ops - m0 < step ? mem_ops - m0 : step;
+#pragma unroll 8
+        for (int32_t k = 0; k < cnt; ++k) acc += buf[k];
+    }
+    uint32_t mix = 0;
+#pragma unroll 4
+    for (int32_t it = sub; it < iters; it += g) mix ^= mix_term(seed, (uint32_t)it);
+    for (int32_t d = g / 2; d > 0; d >>= 1) mix ^= (uint32_t)shfl((int32_t)mix, l ^ d);
+    mix ^= (0x9e3779b9u ^ (uint32_t)node) + sat_u32(acc);
+    if (on && sub == 0) a.out[node] = (double)mix;
 }
 
 }  // namespace tree
@@ -146,7 +188,16 @@ extern "C" int gtap_tree(int32_t height, int32_t mem_ops, int32_t compute_iters,
         return host::invalid_argument("gtap_tree: bad arguments (input_n must be a power of two)");
     tree::NodeArg root{0, height, mem_ops, compute_iters};
     gtap_job job = host::make_job(tree::F_NODE, 0, &root, sizeof(root));
-    tree::TreeArgs a{input, (uint32_t)(input_n - 1), out};
+    // Nodes per batch: a batch of c nodes takes the wave c / 64 of a full one's time, plus the
+    // round's own 4 us or so. Measured (us, caps of 8 / 16 / 32 / 64): 64 reads + 512 steps a node
+    // at height 15: 196 / 221 / 287 / 407, at height 20: 1473 / 1484 / 1577 / 1766; 24 reads +
+    // 160 steps at height 15: 159 / 162 / 179, at height 20: 900 / 757 / 757; 8 reads + 32 steps
+    // at height 15: 148 / 142 / 142 / 157, at height 20: 756 / 527 / 443 / 453. A read counts
+    // like 8 steps; with enough nodes for every wave the round's own time decides.
+    const int64_t node_steps = 8ll * mem_ops + compute_iters;
+    const bool tall = height > 16;
+    const uint32_t batch = node_steps >= 800 ? 8u : (node_steps >= 256 ? (tall ? 16u : 8u) : (tall ? 32u : 16u));
+    tree::TreeArgs a{input, (uint32_t)(input_n - 1), out, batch};
     return host::run_single_job<TreeProgram>(a, job, nullptr, stats, GTAP_TERM_JOBS);
 }
 

@@ -70,6 +70,27 @@ def test_tree_matches_oracle(height, mem_ops, iters):
     assert s["tasks_spawned"] == nodes - 1
 
 
+@pytest.mark.parametrize("height", [0, 2, 3, 6])
+@pytest.mark.parametrize("mem_ops,iters", [(1, 1), (3, 63), (31, 64), (32, 65), (33, 0), (255, 7), (256, 8), (257, 129)])
+def test_tree_lane_groups(height, mem_ops, iters):
+    """A node's reads and steps are divided among 64 / m lanes (m nodes in the round, up to 8
+    here): counts around the groups' step of 4 reads a lane and around whole steps."""
+    print(f"case tree groups height={height} mem_ops={mem_ops} iters={iters}", flush=True)
+    inp = G.tree_input(1 << 12, 7) * 1e6
+    out, _ = G.tree(height, mem_ops, iters, inp)
+    assert np.array_equal(out, O.tree(height, mem_ops, iters, inp))
+
+
+@pytest.mark.parametrize("height,mem_ops,iters", [(16, 2, 8), (17, 2, 8), (16, 32, 0), (17, 32, 0), (17, 20, 640)])
+def test_tree_batch_sizes(height, mem_ops, iters):
+    """One size on each side of the rule that picks 8, 16 or 32 nodes a batch."""
+    print(f"case tree batches height={height} mem_ops={mem_ops} iters={iters}", flush=True)
+    inp = G.tree_input(1 << 16, height)
+    out, s = G.tree(height, mem_ops, iters, inp)
+    assert np.array_equal(out, O.tree(height, mem_ops, iters, inp))
+    assert s["tasks_executed"] == 3 * (1 << height) - 2
+
+
 def test_bfs_on_graph_read_from_reference_format(tmp_path):
     print("case bfs from a CSR file", flush=True)
     row, col = G.rmat_csr(14, 8, 5)
