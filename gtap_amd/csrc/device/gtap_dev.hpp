@@ -40,7 +40,6 @@ enum CtlIndex : int {
                           // counts these, not the launch's worker count: a worker the hardware
                           // has not made resident yet and that owns no job holds no work and
                           // must not be waited for; one that owns a job must)
-    CTL_PROGRAM = 10,     // a counter a program may use (cleared with the others per launch)
     CTL_ARMED = 11,       // 1 after gtap_initialize / gtap_reset: one host-launched entry kernel
                           // may run on this state (it clears the word when it is done)
     CTL_ADMIT_HOLDS = 12, // served: admission attempts the reservation ledger held back
@@ -65,6 +64,7 @@ enum StatIndex : int {
     ST_END_TICKS,    // wall-clock tick at which it left the loop
     ST_RING_SPILLED, // tasks this worker moved from a full deque to the overflow ring
     ST_RING_TAKEN,   // tasks this worker took from the overflow ring
+    ST_PROGRAM,      // this worker's part of the program's count (programs with kLaneSum)
     ST_COUNT = 16
 };
 
@@ -388,6 +388,7 @@ __device__ __forceinline__ int rank_in(uint64_t mask) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 __device__ __forceinline__ int popc(uint64_t m) { return __popcll(m); }
+__device__ __forceinline__ int popc32(uint32_t m) { return __builtin_popcount(m); }
 __device__ __forceinline__ int first_lane(uint64_t m) { return __ffsll((long long)m) - 1; }
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t uniform(uint64_t v) {

@@ -69,6 +69,19 @@ struct HasCoop<P, decltype((void)P::kCoop)> {
     static constexpr bool value = P::kCoop;
 };
 
+// A program may count something over the whole launch (P::kLaneSum): each lane's run() adds to
+// lane.total, and the sums leave with the wave's statistics (ST_PROGRAM), which the summary
+// kernel adds up. One shared counter instead is added to by every round of every wave, and
+// those atomics, all on one line, slow every other memory operation of the launch.
+template <class P, class = void>
+struct HasLaneSum {
+    static constexpr bool value = false;
+};
+template <class P>
+struct HasLaneSum<P, decltype((void)P::kLaneSum)> {
+    static constexpr bool value = P::kLaneSum;
+};
+
 // Most tasks a batch holds: 64, or what the program asks for with its launch arguments
 // (P::batch_cap(args), 1..64). With long task bodies that the whole wave shares (run_coop), a
 // batch of c tasks takes c / 64 of the time of a full one, and the tasks it leaves are
@@ -757,6 +770,7 @@ struct Lane {
     uint32_t outcome;
     bool lds;               // the record's header and first FW frame words are not in HBM yet
     bool sum_join;          // the pending taskwait is an additive join
+    uint32_t total;         // this lane's part of the launch's count (HasLaneSum programs)
     bool coop;              // run_coop finishes this task's body (HasCoop programs)
     int64_t jsum;           // sum of the children's results, after an additive join
     uint64_t join_delta;    // what finishing adds to the parent's join word
@@ -1586,6 +1600,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
     L.rs = pool_rsrc(dev.recs);
     constexpr int QL = CtxShape<P>::kQL;
     const uint32_t bcap = BatchCap<P>::of(args);
+    if constexpr (HasLaneSum<P>::value) L.total = 0u;
 
     uint32_t rng = 0x9E3779B9u ^ (me * 0x85EBCA6Bu) ^ ((uint32_t)lane * 0xC2B2AE35u) ^ (uint32_t)t_begin;
     if (rng == 0) rng = 1;
@@ -2054,6 +2069,12 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         }
     }
 
+    uint64_t program_total = 0;
+    if constexpr (HasLaneSum<P>::value) {
+        program_total = L.total;
+#pragma unroll
+        for (int d = kWave / 2; d > 0; d >>= 1) program_total += shfl(program_total, lane ^ d);
+    }
     if (lane == 0) {
         uint64_t* s = dev.stats + (size_t)me * ST_COUNT;
         s[ST_TASKS] = st.tasks;
@@ -2071,6 +2092,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         s[ST_END_TICKS] = now_ticks();
         s[ST_RING_SPILLED] = vld(&w->ring_spilled);
         s[ST_RING_TAKEN] = st.ring_taken;
+        s[ST_PROGRAM] = program_total;
         if constexpr (Prof) {
             if (dev.prof_phase != nullptr) {
                 uint64_t* ph = dev.prof_phase + (size_t)me * PH_COUNT;

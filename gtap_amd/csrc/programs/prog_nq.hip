@@ -136,44 +136,53 @@ namespace nq {
 
 // The reference's evaluation program at its own settings (evaluation/2-comparison/nq/
 // gtap_nq.cu:10-56): tasks down to row `cutoff`, a sequential search below it, detached
-// spawns (no taskwait) and one shared int32 counter. The sequential search here is an
-// explicit-stack depth-first walk; each task adds its count with one atomic (the reference
-// adds 1 per solution). Unlike the reference, a task that reaches row N counts a solution
-// even above the cutoff, so N <= cutoff + 1 is also correct.
+// spawns (no taskwait) and one count. The sequential search here is a depth-first walk; each
+// lane sums the counts of its tasks, and the sums leave with the wave's statistics at the end
+// of the launch. (The reference adds 1 per solution to one int32. Adding each task's count to
+// one word was bound by that word's line: n = 14 took 752 us, against 500 us without.) Unlike
+// the reference, a task that reaches row N counts a solution even above the cutoff, so
+// N <= cutoff + 1 is also correct.
 struct CutoffArgs {
     int32_t n;
     int32_t cutoff;
-    int32_t* answer;
 };
 
+// Solutions below (row, cols, left, right), row < n: a depth-first walk that lives in registers.
+// The two diagonal sets are kept in board coordinates (bit col - row + n - 1 and bit
+// col + row, at most bit 30 for n <= 16), so a step back is the same exclusive or as the step
+// forward, and the columns of the path are 4 bits each in one 64-bit word: no stack in memory
+// (with one, as four private arrays, every step waited for scratch memory and the walks of a
+// round took 113 us at n = 15). After a step back the columns not yet tried are those above the
+// one taken back. Placements in row n - 2 are not stepped into: the last row's free columns
+// are counted from there.
 __device__ __forceinline__ int32_t nq_serial(int32_t row, int32_t n, uint32_t cols, uint32_t left, uint32_t right) {
-    const uint32_t mask = (n < 32) ? ((1u << n) - 1u) : 0xFFFFFFFFu;
-    uint32_t avail[kMaxN + 1], cs[kMaxN + 1], ls[kMaxN + 1], rs[kMaxN + 1];
-    int32_t count = 0;
-    int32_t d = 0;
-    cs[0] = cols;
-    ls[0] = left;
-    rs[0] = right;
-    avail[0] = mask & ~(cols | left | right);
-    if (row == n) return 1;
-    while (d >= 0) {
-        const uint32_t a = avail[d];
-        if (a == 0u) {
-            --d;
-            continue;
+    const uint32_t mask = (1u << n) - 1u;
+    uint32_t avail = mask & ~(cols | left | right);
+    if (row == n - 1) return popc32(avail);
+    const int32_t top = n - 1;
+    uint32_t dl = (left & mask) << (top - row), dr = (right & mask) << row;
+    uint64_t path = 0;
+    int32_t r = row, count = 0;
+    while (true) {
+        const bool fwd = avail != 0u;
+        if (!fwd && r == row) break;
+        const int32_t at = fwd ? r : r - 1;  // the row whose queen is placed or taken back
+        const uint32_t c = fwd ? (uint32_t)__builtin_ctz(avail | 0x80000000u) : (uint32_t)path & 15u;
+        const uint32_t p = 1u << c;
+        const uint32_t cols1 = cols ^ p, dl1 = dl ^ (p << (top - at)), dr1 = dr ^ (p << at);
+        const int32_t r1 = fwd ? r + 1 : at;
+        const uint32_t free1 = mask & ~(cols1 | (dl1 >> (top - r1)) | (dr1 >> r1));
+        if (fwd && r1 == top) {
+            count += popc32(free1);
+            avail ^= p;
+        } else {
+            cols = cols1;
+            dl = dl1;
+            dr = dr1;
+            r = r1;
+            path = fwd ? (path << 4) | c : path >> 4;
+            avail = fwd ? free1 : free1 & (~1u << c);
         }
-        const uint32_t p = a & (0u - a);
-        avail[d] = a - p;
-        if (row + d + 1 == n) {
-            ++count;
-            continue;
-        }
-        const uint32_t c = cs[d] | p, l = (ls[d] | p) << 1, r = (rs[d] | p) >> 1;
-        ++d;
-        cs[d] = c;
-        ls[d] = l;
-        rs[d] = r;
-        avail[d] = mask & ~(c | l | r);
     }
     return count;
 }
@@ -181,7 +190,8 @@ __device__ __forceinline__ int32_t nq_serial(int32_t row, int32_t n, uint32_t co
 struct CutoffProgram {
     static constexpr int kQueues = 1;
     static constexpr bool kNoTaskwait = true;
-    static constexpr int kWavesPerSimd = 3;
+    static constexpr bool kLaneSum = true;
+    static constexpr int kWavesPerSimd = 4;
     static constexpr int kFrameWords = 4;  // row, cols, left, right
     static constexpr uint32_t kMaxFunc = F_NQ;
     static constexpr uint32_t kFrameBytes = 16;
@@ -207,7 +217,7 @@ struct CutoffProgram {
                 __gtap_spawn_task_detached(lane, F_NQ, 0, NqArg{row + 1, cols | p, (left | p) << 1, (right | p) >> 1});
             }
         }
-        if (found) atomic_add(g.answer, found);
+        lane.total += (uint32_t)found;
         __gtap_finish_task(lane);
     }
 };
@@ -246,7 +256,7 @@ extern "C" int gtap_nqueens_slots(int n, int64_t* result, gtap_run_stats* stats)
 
 // The reference's n-queens benchmark at its own settings (evaluation/2-comparison/nq/
 // gtap_nq.cu:57-99): tasks for rows 0..cutoff (the reference's default 7), a sequential search
-// below, no taskwait, one int32 counter. Returns the solution count in *result.
+// below, no taskwait, one count. Returns the solution count in *result.
 extern "C" int gtap_nqueens_cutoff(int n, int cutoff, int64_t* result, gtap_run_stats* stats) {
     using namespace gtap;
     if (n < 1 || n > nq::kMaxN || cutoff < 0) return host::invalid_argument("gtap_nqueens_cutoff: n in [1, 16], cutoff >= 0");
@@ -255,15 +265,11 @@ extern "C" int gtap_nqueens_cutoff(int n, int cutoff, int64_t* result, gtap_run_
         int st = gtap_initialize();
         if (st) return st;
     }
-    // the counter: the launch's program control word, cleared by the per-launch reset
-    int32_t* answer = R.ctl + CTL_PROGRAM * 32;
     nq::NqArg root{0, 0u, 0u, 0u};
     gtap_job job = host::make_job(nq::F_NQ, 0, &root, sizeof(root));
-    int st = host::run_single_job<gtap::nq::CutoffProgram>(nq::CutoffArgs{n, cutoff, answer}, job, nullptr, stats,
+    int st = host::run_single_job<gtap::nq::CutoffProgram>(nq::CutoffArgs{n, cutoff}, job, nullptr, stats,
                                                             GTAP_TERM_QUIESCE);
     if (st) return st;
-    int32_t v = 0;
-    GTAP_HIP_TRY(hipMemcpy(&v, answer, sizeof(v), hipMemcpyDeviceToHost));
-    if (result) *result = v;
+    if (result) *result = (int64_t)R.summary->sums[ST_PROGRAM];
     return 0;
 }

@@ -92,7 +92,9 @@ int gtap_get_last_stats(gtap_run_stats* out);
 /* Per-wave counters of the last launch: 16 uint64 per worker, in the order tasks executed,
  * tasks spawned, rounds, pops, steals, steal attempts, jobs admitted, pool refills, records
  * published, records pushed out of the LDS window, suspended taskwaits, the 100 MHz
- * wall-clock ticks at which the worker started and stopped, then 3 unused. */
+ * wall-clock ticks at which the worker started and stopped, tasks moved to and taken from the
+ * overflow ring, and the worker's part of the program's count (n-queens with a cutoff: the
+ * solutions it found; else 0). */
 int gtap_get_worker_stats(uint64_t* out, uint32_t max_workers, uint32_t* nworkers_out);
 int gtap_device_info(char* name, int name_len, int* num_cus, uint64_t* hbm_bytes);
 
@@ -202,7 +204,7 @@ int gtap_stream_set_merge_leaf(gtap_stream* stream, int32_t merge_leaf);
 
 /* n-queens at the reference's benchmark settings (evaluation/2-comparison/nq/gtap_nq.cu:10-99):
  * tasks for rows 0..cutoff (the reference uses 7), a sequential search below, detached
- * spawns, one int32 counter. */
+ * spawns, one count. */
 int gtap_nqueens_cutoff(int n, int cutoff, int64_t* result, gtap_run_stats* stats);
 
 /* Block-mode BFS (examples/asynchronous_bfs/asynchronous_bfs_block.cu:17-37): one vertex
