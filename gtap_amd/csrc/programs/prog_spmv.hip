@@ -10,7 +10,7 @@
 //       y[i] = sum;
 //   }
 //   #pragma gtap function
-//   __device__ void range_spmv(int begin, int end) {
+//   __device__ void range_spmv(int begin, int end) {          // (in 4 pieces here)
 //       if (end - begin <= CUTOFF) {
 //           for (int i = begin; i < end; ++i) {
 //               #pragma gtap task
@@ -54,22 +54,38 @@ struct SpmvArgs {
     int32_t rows;
     int32_t cols;
     int32_t cutoff;
+    uint32_t batch;   // most tasks a wave takes at once
+    int32_t fan;      // pieces a range is cut into
     int32_t nnz;  // row_ptr[rows]: a row's offsets must satisfy 0 <= row_ptr[i] <= row_ptr[i+1] <= nnz
 };
+
+constexpr int kPer = 8;        // entries of a row that a lane loads in one step
+constexpr int kGroup = 8;      // most lanes per row while there are rows for all lanes
+constexpr int kRowBegin = 2;   // frame words a row task keeps its offsets in
+constexpr int kRowLength = 3;
+typedef double Entry __attribute__((ext_vector_type(2)));  // a value and its x entry
 
 struct Program {
     static constexpr int kQueues = 1;
     static constexpr bool kNoTaskwait = true;  // detached spawns only
+    static constexpr bool kCoop = true;        // the rows of a round are summed by run_coop
+    static constexpr int kWavesPerSimd = 2;    // what the tile's LDS allows; 3 with kPer = 4: 4.26 against 4.01 ms
     static constexpr int kFrameWords = 2;      // begin, end (a row task uses begin)
     static constexpr uint32_t kMaxFunc = F_ROW;
     static constexpr uint32_t kFrameBytes = 16;
     using Args = SpmvArgs;
+    struct WaveShared {
+        Entry tile[kWave * kPer + kWave];  // kWave / g rows of kPer * g entries, each row padded by one
+        int32_t src[kWave];                // lanes that hold the round's rows
+    };
+    __device__ __forceinline__ static uint32_t batch_cap(const Args& a) { return a.batch; }
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
+    template <class L>
+    __device__ __forceinline__ static void run_coop(L& lane, uint64_t mask, WaveShared* sh);
 };
 
-// One row: the column indices and values of 8 entries are loaded together, then their x
-// entries, then the fma chain runs in column order.
+// A row task checks its row's offsets and leaves the entries to run_coop.
 template <class L>
 __device__ __forceinline__ void row_task(L& lane) {
     const SpmvArgs& g = *lane.args;
@@ -85,31 +101,9 @@ __device__ __forceinline__ void row_task(L& lane) {
         __gtap_finish_task(lane);
         return;
     }
-    double sum = 0.0;
-    constexpr int kChunk = 8;
-    for (int32_t b = kb; b < ke; b += kChunk) {
-        int32_t c[kChunk];
-        double v[kChunk];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            c[j] = (b + j < ke) ? g.col_idx[b + j] : 0;
-            v[j] = (b + j < ke) ? g.val[b + j] : 0.0;
-        }
-        bool bad = false;
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) bad |= (b + j < ke) && (c[j] < 0 || c[j] >= g.cols);
-        if (bad) {
-            GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, i, g.cols);
-            break;
-        }
-        double xv[kChunk];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) xv[j] = (b + j < ke) ? g.x[c[j]] : 0.0;
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-            if (b + j < ke) sum = __builtin_fma(v[j], xv[j], sum);
-    }
-    g.y[i] = sum;
+    lane.frame[kRowBegin] = (uint32_t)kb;
+    lane.frame[kRowLength] = (uint32_t)(ke - kb);
+    lane.coop = true;
     __gtap_finish_task(lane);
 }
 
@@ -121,11 +115,126 @@ __device__ __forceinline__ void range_task(L& lane) {
     if (end - begin <= g.cutoff) {
         for (int32_t i = begin; i < end; ++i) __gtap_spawn_task_detached(lane, F_ROW, 0, RangeArg{i, 0});
     } else {
-        const int32_t mid = (begin + end) >> 1;
-        __gtap_spawn_task_detached(lane, F_RANGE, 0, RangeArg{begin, mid});
-        __gtap_spawn_task_detached(lane, F_RANGE, 0, RangeArg{mid, end});
+        const int64_t len = (int64_t)end - begin;
+        for (int32_t i = 0; i < g.fan; ++i) {
+            const int32_t ps = begin + (int32_t)(len * i / g.fan), pe = begin + (int32_t)(len * (i + 1) / g.fan);
+            if (pe > ps) __gtap_spawn_task_detached(lane, F_RANGE, 0, RangeArg{ps, pe});
+        }
     }
     __gtap_finish_task(lane);
+}
+
+// The entries of the kPer * g of a row's entries that one step takes: this lane's columns and
+// values, entry j at offset first + j * g of a row of `length` entries from `begin`.
+__device__ __forceinline__ void load_entries(const SpmvArgs& a, int32_t begin, int32_t length, int32_t first, int32_t g,
+                                             int32_t (&c)[kPer], double (&v)[kPer]) {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int32_t e = first + j * g;
+        c[j] = e < length ? __builtin_nontemporal_load(a.col_idx + begin + e) : -1;
+        v[j] = e < length ? __builtin_nontemporal_load(a.val + begin + e) : 0.0;
+    }
+}
+
+// The rows of a round on all 64 lanes. One lane per row reads 64 separate lines with every
+// load, uses 4 or 8 bytes of each and has lost them from the caches when it comes back, and a
+// round lasts as long as its longest row: 6.6 ms for 1M rows of 300 entries (345 M lines from
+// beyond the L2). Here g lanes load a row's entries together, kPer each per step: whole lines of
+// columns and values are used at once and not kept (non-temporal), and the entries
+// {value, x[column]} go through LDS to one lane per row, which runs the row's chain of fused
+// multiply-adds in column order, so the sum has the same bits. g is the smallest power of two
+// with kPer * g entries for the longest row, at most kGroup (4 / 8 / 16 with full batches: 4.55 /
+// 4.01 / 3.95 ms at 300 entries a row, 409 / 395 / 428 us at 100) unless fewer rows leave lanes
+// free. 3.72 ms, 1.02 TB/s of matrix: bound by the gathers of x (8 MB against 4 MB of L2 per
+// XCD), 215 M lines at 58 G/s, about the rate of random reads that miss the L2 on this chip.
+template <class L>
+__device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
+    const SpmvArgs& a = *lane.args;
+    const int32_t l = lane_id();
+    const int32_t m = popc(mask);
+    int32_t longest = lane.coop ? (int32_t)lane.frame[kRowLength] : 0;
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        const int32_t o = shfl(longest, l ^ d);
+        longest = o > longest ? o : longest;
+    }
+    int32_t g = 1;
+    while (kPer * g < longest && (g < kGroup || 2 * g * m <= kWave) && g < kWave) g <<= 1;
+    if (lane.coop) lds(sh->src)[rank_in(mask)] = l;
+    wave_sync();
+    const int32_t rows = kWave / g, step = kPer * g, stride = step + 1;
+    const int32_t slot = l / g, sub = l & (g - 1);
+    lds_array<Entry> tile = lds(sh->tile);
+    // The steps of all groups in one sequence, the next step's columns and values in flight
+    // while the current one gathers and sums, over the end of a group too.
+    int32_t p0 = 0, b = 0;       // current step: the group's first row (of the m), its entries' offset
+    int32_t begin, length;       // this lane loads entries sub, sub + g, ... of row p0 + slot
+    int32_t row, left;           // and, among the first `rows` lanes, sums row p0 + l: entries left
+    bool sums;
+    auto load_part = [&](int32_t p) {
+        const bool on = p + slot < m;
+        const int32_t src = lds(sh->src)[on ? p + slot : 0];
+        begin = shfl((int32_t)lane.frame[kRowBegin], src);
+        length = shfl((int32_t)lane.frame[kRowLength], src);
+        if (!on) length = 0;
+    };
+    auto sum_part = [&](int32_t p) {
+        sums = l < rows && p + l < m;
+        const int32_t own = lds(sh->src)[sums ? p + l : 0];
+        row = shfl((int32_t)lane.frame[0], own);
+        left = shfl((int32_t)lane.frame[kRowLength], own);
+        if (!sums) left = 0;
+    };
+    load_part(0);
+    sum_part(0);
+    double sum = 0.0;
+    int32_t c[kPer];
+    double v[kPer];
+    load_entries(a, begin, length, sub, g, c, v);
+    while (true) {
+        double xv[kPer];
+        bool bad = false;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const bool in = b + j * g + sub < length;
+            const bool valid = (uint32_t)c[j] < (uint32_t)a.cols;
+            bad |= in && !valid;
+            xv[j] = in && valid ? a.x[c[j]] : 0.0;
+        }
+        if (bad) GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, begin, a.cols);
+        const bool more = ballot(b + step < length) != 0;
+        b = more ? b + step : 0;
+        const int32_t p1 = more ? p0 : p0 + rows;
+        if (!more && p1 < m) load_part(p1);
+        int32_t c1[kPer];
+        double v1[kPer];
+        if (p1 < m) load_entries(a, begin, length, b + sub, g, c1, v1);
+        wave_sync();  // the previous step's entries have been read
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) tile[slot * stride + j * g + sub] = Entry{v[j], xv[j]};
+        wave_sync();
+        for (int32_t e = 0; e < step && e < left; e += kPer) {
+            Entry t[kPer];
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) t[j] = tile[l * stride + e + j];
+#pragma unroll
+            for (int j = 0; j < kPer; ++j)
+                if (e + j < left) sum = __builtin_fma(t[j].x, t[j].y, sum);
+        }
+        left -= step;
+        if (!more) {
+            if (sums) a.y[row] = sum;
+            if (p1 >= m) break;
+            sum = 0.0;
+            sum_part(p1);
+        }
+        p0 = p1;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            c[j] = c1[j];
+            v[j] = v1[j];
+        }
+    }
 }
 
 template <class L>
@@ -158,9 +267,23 @@ extern "C" int gtap_spmv(const int32_t* row_ptr, const int32_t* col_idx, const d
     GTAP_HIP_TRY(hipMemcpy(&nnz, row_ptr + rows, sizeof(int32_t), hipMemcpyDeviceToHost));
     if (nnz < 0) return host::invalid_argument("gtap_spmv: negative entry count");
     if (nnz > 0 && (!col_idx || !val)) return host::invalid_argument("gtap_spmv: bad arguments");
+    if (int st = gtap_initialize()) return st;
     spmv::RangeArg root{0, rows};
     gtap_job job = host::make_job(spmv::F_RANGE, 0, &root, sizeof(root));
-    spmv::SpmvArgs a{row_ptr, col_idx, val, x, y, rows, cols, cutoff, nnz};
+    spmv::SpmvArgs a{row_ptr, col_idx, val, x, y, rows, cols, cutoff, 64u, 2, nnz};
+    // Rows per batch, by the mean row length: a batch's time is its entries', so with long rows
+    // small batches spread better, and with short ones the round's own time counts. Measured (us,
+    // batches of 64 / 32 / 16 / 8, ranges cut in 4): 1M rows of 300: 3870 / 3784 / 3737 / 3722;
+    // 5000 rows of 200: 215 / 146 / 142 / 140; 200003 rows of 100: 363 / 328 / 332 / 358; 512K rows
+    // of 40: 402 / 384 / 412 / 481; 1M rows of 5: 336 / 334 / 403 / 573. Ranges cut in 4 instead of
+    // 2 reach full batches in half the rounds (1000 rows of 10: 83 -> 77 us). A cutoff whose full
+    // batch of ranges does not fit the deque keeps full batches of halves: it ends in the
+    // queue-overflow error as it always has.
+    if (64ll * cutoff <= (int64_t)host::rt().cap - (int64_t)kMargin) {
+        const int64_t mean = nnz / rows;
+        a.batch = mean >= 160 ? 8u : (mean >= 96 ? 16u : 32u);
+        a.fan = 4;
+    }
     return host::run_single_job<SpmvProgram>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
 }
 

@@ -58,6 +58,37 @@ def test_spmv_empty_rows_and_zero_matrix():
     assert np.all(y0 == 0.0)
 
 
+@pytest.mark.parametrize("lengths", [[0, 1, 7, 8, 9], [15, 16, 17, 31, 32, 33], [63, 64, 65, 127, 128, 129],
+                                     [511, 512, 513, 1, 0], [5000], [0], [100, 3] * 40, [300] * 70, [1] * 1000])
+@pytest.mark.parametrize("cutoff", [1, 16, 500])
+def test_spmv_row_lengths(lengths, cutoff):
+    """Rows whose lengths meet the edges of a step (8 entries for each of a row's 1 to 64 lanes),
+    few and many in a batch, and the batch sizes of short and long mean rows."""
+    print(f"case spmv lengths {lengths[:6]} x {len(lengths)} cutoff={cutoff}", flush=True)
+    rng = np.random.default_rng(len(lengths) + cutoff)
+    cols = max(max(lengths), 40)
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(cols, k, replace=False)) for k in lengths] + [[]]).astype(np.int32)
+    va = rng.uniform(-1, 1, ci.size)
+    x = rng.uniform(-2, 2, cols)
+    x[0] = np.inf  # an entry that no row uses by accident: padding must not be multiplied in
+    ci[ci == 0] = 1
+    y, _ = G.spmv(rp, ci, va, x, cutoff)
+    assert np.array_equal(y, O.spmv(rp, ci, va, x))
+
+
+def test_spmv_bad_column_is_reported():
+    print("case spmv bad column", flush=True)
+    rp, ci, va = G.spmv_random(500, 30, 3)
+    for bad in (-1, 500, 2**31 - 1):
+        c = ci.copy()
+        c[len(c) // 2] = bad
+        with pytest.raises(G.GtapError) as e:
+            G.spmv(rp, c, va, np.ones(500))
+        assert "INVALID_ARGUMENT" in str(e.value)
+    assert np.array_equal(G.spmv(rp, ci, va, np.ones(500))[0], O.spmv(rp, ci, va, np.ones(500)))
+
+
 @pytest.mark.parametrize("height,mem_ops,iters", [(0, 4, 4), (1, 0, 0), (5, 64, 512), (10, 16, 32), (15, 64, 512),
                                                   (12, 0, 1000)])
 def test_tree_matches_oracle(height, mem_ops, iters):
