@@ -82,6 +82,23 @@ struct HasLaneSum<P, decltype((void)P::kLaneSum)> {
     static constexpr bool value = P::kLaneSum;
 };
 
+// Victims an idle wave probes per steal attempt once kPatientAfter attempts in a row have found
+// nothing: all of gtap_config.probe_lanes, or P::kIdleProbes if that is fewer. At launch start and
+// end thousands of waves are idle, and 8 lines each every 1.3 us is nearly half of the random
+// reads the memory serves; programs whose rounds are bound by memory run faster with 2, those of
+// short dependent rounds find work later with fewer than 8. Measured with 8 / 2 (us): R-MAT 18
+// BFS 388 / 279, n-queens(13) with a cutoff 343 / 263, SpMV of 20011 rows 125 / 109; but n-queens(12)
+// 197 / 201, the tree of height 15 191 / 205.
+template <class P, class = void>
+struct IdleProbes {
+    static constexpr uint32_t value = kWave;
+};
+template <class P>
+struct IdleProbes<P, decltype((void)P::kIdleProbes)> {
+    static constexpr uint32_t value = P::kIdleProbes;
+};
+constexpr uint32_t kPatientAfter = 8;
+
 // Most tasks a batch holds: 64, or what the program asks for with its launch arguments
 // (P::batch_cap(args), 1..64). With long task bodies that the whole wave shares (run_coop), a
 // batch of c tasks takes c / 64 of the time of a full one, and the tasks it leaves are
@@ -1278,18 +1295,18 @@ __device__ __forceinline__ uint32_t pick_victim(const GtapDev& dev, uint32_t me,
 }
 
 // With several EPAQ queues, one probe of every queue at once: lane l probes queue
-// (cq + l) % Q of a random victim (probe_lanes victims per queue, at most 64 probes), and one
+// (cq + l) % Q of a random victim (nprobe victims per queue, at most 64 probes), and one
 // CAS claims up to half (<= steal_batch; 1 on the wave queue) of a non-empty one. The thief
 // finds work in one round trip instead of one per queue. Returns the number stolen into
 // `tid_out` and the queue in `q_out`.
 template <class P>
 __device__ __forceinline__ uint32_t try_steal_any(const GtapDev& dev, uint32_t me, uint32_t cq, uint32_t& rng,
                                                   uint32_t& tid_out, bool& idle_registered, LoopStats& st,
-                                                  uint32_t& q_out, uint32_t max_items) {
+                                                  uint32_t& q_out, uint32_t max_items, uint32_t nprobe) {
     constexpr uint32_t Q = (uint32_t)P::kQueues;
     const int lane = lane_id();
     if (dev.nworkers < 2) return 0;
-    uint32_t probes = dev.probe_lanes * Q;
+    uint32_t probes = nprobe * Q;
     if (probes > (uint32_t)kWave) probes = kWave;
     uint32_t victim = 0, q = (cq + (uint32_t)lane) % Q;
     uint64_t wv = 0;
@@ -1336,7 +1353,7 @@ __device__ __forceinline__ uint32_t try_steal_any(const GtapDev& dev, uint32_t m
 template <class P>
 __device__ __forceinline__ uint32_t try_steal(const GtapDev& dev, uint32_t me, uint32_t q, uint32_t& rng,
                                               uint32_t& tid_out, bool& idle_registered, LoopStats& st,
-                                              uint32_t max_items = kWave) {
+                                              uint32_t max_items, uint32_t nprobe) {
     uint32_t batch_cap = ((int)q == HasWaveQueue<P>::value) ? 1u : dev.steal_batch;
     if (batch_cap > max_items) batch_cap = max_items;
     const int lane = lane_id();
@@ -1344,7 +1361,7 @@ __device__ __forceinline__ uint32_t try_steal(const GtapDev& dev, uint32_t me, u
     uint32_t victim = 0;
     uint64_t wv = 0;
     int32_t sz = 0;
-    if ((uint32_t)lane < dev.probe_lanes) {
+    if ((uint32_t)lane < nprobe) {
         victim = pick_victim(dev, me, rng, lane);
         wv = ld64(dq_word_ptr(dev, q, victim));
         sz = (int32_t)((uint32_t)wv - (uint32_t)(wv >> 32));
@@ -1380,38 +1397,51 @@ __device__ __forceinline__ uint32_t try_steal(const GtapDev& dev, uint32_t me, u
 }
 
 // Pop up to 64 (max_items) of this wave's newest published tasks from queue q. The queue must
-// hold no private entries (its tail equals its bottom): both move to the new bottom.
+// hold no private entries (its tail equals its bottom): both move to the new bottom. The owner
+// knows the bottom and a lower bound of the top, so it starts with a CAS on the word it
+// expects, and reads its slots, which only it writes, while the CAS is under way: one round trip
+// where a load of the word, the CAS and the slot loads took three. A theft since the last look
+// makes the CAS fail and return the word.
 template <class P>
 __device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, WaveCtxOf<P>* w, uint32_t me, uint32_t q,
                                             uint32_t& tid_out, uint32_t max_items = kWave) {
     const int lane = lane_id();
     uint64_t* wp = dq_word_ptr(dev, q, me);
+    const uint32_t b = uniform(vld(&w->bottom[q]));
+    uint32_t t = uniform(vld(&w->top_cache[q]));
+    uint32_t cap = ((int)q == HasWaveQueue<P>::value) ? 1u : (uint32_t)kWave;
+    if (cap > max_items) cap = max_items;
+    uint32_t k0 = 0;   // the number of slots read: positions [b - k0, b)
+    uint32_t tid = 0;
     // A failed CAS means a thief took tasks, so this ends; the owner leaves with a task or an
     // empty deque. Only the owner pushes, so the deque stays empty while the owner is idle
     // (idle waves do not pop again, and quiescence may count them idle).
     while (true) {
-        uint64_t wv = 0;
-        if (lane == 0) wv = ld64(wp);
-        wv = shfl(wv, 0);
-        const uint32_t t = (uint32_t)(wv >> 32), b = (uint32_t)wv;
         const int32_t sz = (int32_t)(b - t);
-        if (sz <= 0) return 0;
-        uint32_t cap = ((int)q == HasWaveQueue<P>::value) ? 1u : (uint32_t)kWave;
-        if (cap > max_items) cap = max_items;
-        const uint32_t k = (uint32_t)sz < cap ? (uint32_t)sz : cap;
-        int ok = 0;
-        if (lane == 0) {
-            uint64_t expected = wv;
-            ok = atomic_cas(wp, expected, ((uint64_t)t << 32) | (uint64_t)(b - k)) ? 1 : 0;
+        if (sz <= 0) {
+            if (lane == 0) vst(&w->top_cache[q], t);
+            return 0;
         }
+        const uint32_t k = (uint32_t)sz < cap ? (uint32_t)sz : cap;
+        if (k0 == 0) {
+            k0 = k;
+            if ((uint32_t)lane < k) tid = ld32(dq_slot_ptr(dev, q, me, b - k + (uint32_t)lane));
+        }
+        uint64_t seen = ((uint64_t)t << 32) | (uint64_t)b;
+        int ok = 0;
+        if (lane == 0) ok = atomic_cas(wp, seen, ((uint64_t)t << 32) | (uint64_t)(b - k)) ? 1 : 0;
         ok = shfl((int32_t)ok, 0);
         if (ok) {
-            if ((uint32_t)lane < k) tid_out = ld32(dq_slot_ptr(dev, q, me, b - k + (uint32_t)lane));
-            vst(&w->bottom[q], b - k);
-            vst(&w->tail[q], b - k);
-            vst(&w->top_cache[q], t);
+            if (k != k0) tid = shfl(tid, lane + (int)(k0 - k));  // fewer than read: the newest k
+            tid_out = tid;
+            if (lane == 0) {
+                vst(&w->bottom[q], b - k);
+                vst(&w->tail[q], b - k);
+                vst(&w->top_cache[q], t);
+            }
             return k;
         }
+        t = (uint32_t)(shfl(seen, 0) >> 32);
     }
 }
 
@@ -1666,17 +1696,19 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                 st.jobs += n;
                 batch_q = -1;
             }
+            const uint32_t nprobe = idle_iter >= kPatientAfter && IdleProbes<P>::value < dev.probe_lanes
+                                        ? IdleProbes<P>::value : dev.probe_lanes;
             if (n == 0) {
                 if constexpr (kStealAnyQueue && Sched == kSchedWS && Q > 1) {
                     uint32_t sq = 0;
-                    n = try_steal_any<P>(dev, me, cq, rng, my_tid, idle_registered, st, sq, bcap);
+                    n = try_steal_any<P>(dev, me, cq, rng, my_tid, idle_registered, st, sq, bcap, nprobe);
                     if (n) batch_q = (int)sq;
                 } else {
 #pragma unroll
                     for (int i = 0; i < Q && n == 0; ++i) {
                         const uint32_t q = (cq + (uint32_t)i) % (uint32_t)Q;
                         if constexpr (Sched == kSchedGQ) n = gq_pop<P>(dev, q, my_tid, idle_registered, st);
-                        else n = try_steal<P>(dev, me, q, rng, my_tid, idle_registered, st, Sched == kSchedCL ? 1u : bcap);
+                        else n = try_steal<P>(dev, me, q, rng, my_tid, idle_registered, st, Sched == kSchedCL ? 1u : bcap, nprobe);
                         if (n) batch_q = (int)q;
                     }
                 }

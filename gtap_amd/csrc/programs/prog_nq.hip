@@ -190,6 +190,7 @@ __device__ __forceinline__ int32_t nq_serial(int32_t row, int32_t n, uint32_t co
 struct CutoffProgram {
     static constexpr int kQueues = 1;
     static constexpr bool kNoTaskwait = true;
+    static constexpr uint32_t kIdleProbes = 2;
     static constexpr bool kLaneSum = true;
     static constexpr int kWavesPerSimd = 4;
     static constexpr int kFrameWords = 4;  // row, cols, left, right

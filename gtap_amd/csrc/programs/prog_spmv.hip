@@ -68,6 +68,7 @@ typedef double Entry __attribute__((ext_vector_type(2)));  // a value and its x 
 struct Program {
     static constexpr int kQueues = 1;
     static constexpr bool kNoTaskwait = true;  // detached spawns only
+    static constexpr uint32_t kIdleProbes = 2;
     static constexpr bool kCoop = true;        // the rows of a round are summed by run_coop
     static constexpr int kWavesPerSimd = 2;    // what the tile's LDS allows; 3 with kPer = 4: 4.26 against 4.01 ms
     static constexpr int kFrameWords = 2;      // begin, end (a row task uses begin)
