@@ -20,7 +20,7 @@
 //           int u = col[i];
 //           if (atomicMin(&depth[u], d + 1) > d + 1) {
 //               #pragma gtap task queue(bucket(row[u + 1] - row[u]))
-//               bfs(u, row[u], row[u + 1], d + 1);
+//               bfs(u, row[u], row[u + 1], d + 1);   // (not for a u without out-edges)
 //           }
 //       }
 //   }
@@ -30,9 +30,8 @@
 // launch ends by quiescence. Distances are the BFS hop counts whatever the schedule.
 //
 // With 4 queues, queue 3 (ranges of 512 edges and more) is a wave queue: its task runs on a
-// whole wavefront, which reads the range 512 edges at a time (lane l takes edges b + l + 64 j,
-// so each column load is one contiguous 256-byte read) and spawns every improved neighbour
-// from the lane that found it. A range above kWaveSplitEdges (or an eighth of the deque
+// whole wavefront, which scans the range 512 edges at a time as a round's lane tasks are
+// (expand, below). A range above kWaveSplitEdges (or an eighth of the deque
 // capacity, if smaller) is first cut into up to 64 near-equal pieces, one spawned per lane.
 // A hub's adjacency list is thus scanned by a few wave rounds instead of a tree of 64-edge
 // lane tasks and their split tasks. One queue keeps the lane program for every range. (The
@@ -67,23 +66,44 @@ __host__ __device__ __forceinline__ uint32_t degree_bucket(int32_t deg) {
 
 constexpr int32_t kSplitFanout = 8;         // pieces per split of a lane task's range
 constexpr int32_t kWaveSplitEdges = 2048;  // a wave task scans at most this many edges (and cap / 8)
-constexpr int kWaveChunk = 8;               // edges per lane per step of a wave scan
+constexpr int kWindows = 8;                 // edges per lane per step of an expansion
+constexpr int kHits = 192;                  // improved vertices held before their tasks are spawned
+
+struct Segment {   // one task's edges in the flat sequence of a round's edges
+    int32_t shift; // flat edge f is column entry f + shift
+    int32_t nd;    // depth its neighbours get
+};
+struct Hit {
+    int32_t u;
+    int32_t nd;
+};
+struct ExpandShared {
+    uint32_t starts[2 * kWindows];  // per window of 64 flat edges, which of them start a segment
+    Segment seg[kWave];
+    Hit hit[kHits];
+};
 
 template <int NQ>
 struct Program {
     static constexpr int kQueues = NQ;
     static constexpr int kWaveQueue = NQ == 4 ? 3 : -1;
     static constexpr bool kNoTaskwait = true;  // detached spawns only
+    static constexpr uint32_t kIdleProbes = 2;
     static constexpr int kWavesPerSimd = 3;    // 3072 wavefront workers with 4 queues too (4 per SIMD measured slower)
     static constexpr int kFrameWords = 4;
     static constexpr uint32_t kMaxFunc = F_BFS;
     static constexpr uint32_t kFrameBytes = 16;
     using Args = BfsArgs;
-    struct WaveShared {
-        int32_t unused;
-    };
+    using WaveShared = ExpandShared;
+    static constexpr bool kCoop = true;  // the edges of a round are scanned by run_coop
+    // With one queue a wave holds few tasks while the search spreads, and 32 a batch spread it
+    // sooner: R-MAT 18, 64 / 32 / 16 a batch: 297 / 258 / 286 us, R-MAT 22: 1050 / 1048 / 1288 us. With
+    // four, each queue's batch is smaller anyway: R-MAT 22, 64 / 32: 1116 / 1196 us.
+    __device__ __forceinline__ static uint32_t batch_cap(const Args&) { return NQ == 1 ? 32u : 64u; }
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
+    template <class L>
+    __device__ __forceinline__ static void run_coop(L& lane, uint64_t mask, WaveShared* sh);
     template <class W>
     __device__ __forceinline__ static void run_wave(W& wt);
 };
@@ -97,82 +117,144 @@ __device__ __forceinline__ uint32_t route(int32_t deg) {
     }
 }
 
-template <int NQ, class L>
-__device__ __forceinline__ void bfs_task(L& lane) {
-    const BfsArgs& g = *lane.args;
-    const int32_t v = lane.template arg<int32_t>(0);
-    const int32_t s = lane.template arg<int32_t>(4);
-    const int32_t e = lane.template arg<int32_t>(8);
-    const int32_t d = lane.template arg<int32_t>(12);
-    if (ld32(reinterpret_cast<const int32_t*>(g.depth) + v) < d) {  // stale: v was reached by a shorter path meanwhile
-        __gtap_finish_task(lane);
-        return;
-    }
-    if (e - s > g.split) {
-        // up to kSplitFanout near-equal pieces, each routed by its own length
-        const int64_t len = (int64_t)e - s;
-        int32_t k = (int32_t)((len + g.split - 1) / g.split);
-        if (k > kSplitFanout) k = kSplitFanout;
-        for (int32_t i = 0; i < k; ++i) {
-            const int32_t ps = s + (int32_t)(len * i / k);
-            const int32_t pe = s + (int32_t)(len * (i + 1) / k);
-            __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
+template <class P>
+__device__ __forceinline__ void spawn_one(Lane<P>& t, uint32_t f, uint32_t q, const BfsArg& a) {
+    __gtap_spawn_task_detached(t, f, q, a);
+}
+template <class P>
+__device__ __forceinline__ void spawn_one(WaveTask<P>& t, uint32_t f, uint32_t q, const BfsArg& a) {
+    t.spawn_detached_lane(f, q, a);
+}
+
+// Spawns the tasks of the `count` improved vertices in sh->hit, one per lane and turn. A vertex
+// without out-edges needs none.
+template <int NQ, class T>
+__device__ __forceinline__ void spawn_hits(T& t, const BfsArgs& g, ExpandShared* sh, int32_t count) {
+    const int32_t l = lane_id();
+    wave_sync();
+    for (int32_t b = 0; b < count; b += kWave) {
+        if (b + l < count) {
+            const int32_t u = lds(sh->hit)[b + l].u, nd = lds(sh->hit)[b + l].nd;
+            const int32_t us = g.row[u], ue = g.row[u + 1];
+            if (us < 0 || ue < us || (int64_t)ue > g.ne)  // malformed offsets: never read past col
+                GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, u, g.nv);
+            else if (ue > us)
+                spawn_one(t, F_BFS, route<NQ>(ue - us), BfsArg{u, us, ue, nd});
         }
-        __gtap_finish_task(lane);
-        return;
     }
-    // Edges in chunks of kChunkEdges: the column loads, the depth probes and the atomicMins of
-    // a chunk are issued back to back, so their latencies overlap instead of adding up edge
-    // by edge. A plain load of depth[u] filters the atomic: depths only decrease, so a stale
-    // cached value is never below the true one and can only cost an unneeded atomic. A chunk
-    // is 16 edges: fewer dependent chains per task than 8 (1.33 -> 1.29 ms with one queue,
-    // 1.43 -> 1.40 ms with four).
-    constexpr int kChunkEdges = 16;
-    const int32_t nd = d + 1;
-    for (int32_t b = s; b < e; b += kChunkEdges) {
-        int32_t u[kChunkEdges];
+    wave_sync();
+}
+
+// Scans a round's edges on all 64 lanes: each lane brings a range of `length` columns from
+// `begin` (none: 0), whose vertices get depth nd. The ranges form one flat sequence of edges and
+// lane l takes edges b + 64 j + l of it, so every lane has work until the last edges, a round
+// lasts as long as its edges and not as its longest range, and loads are contiguous. (With one
+// range per lane, 16 edges at a time, a round of R-MAT 22 took 22.6 us for 717 edges on average,
+// four chains of dependent loads for the longest range.)
+//
+// kWindows column loads per lane are in flight together, then their probes, then their atomics.
+// A plain load of depth[u] filters the atomics: depths only decrease, so a stale cached value is
+// never below the true one and can only cost an unneeded atomic.
+template <int NQ, class T>
+__device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh, int32_t begin, int32_t length,
+                                       int32_t nd_own) {
+    const int32_t l = lane_id();
+    int32_t end = length;  // inclusive prefix sum
 #pragma unroll
-        for (int j = 0; j < kChunkEdges; ++j) u[j] = (b + j < e) ? g.col[b + j] : -1;
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int32_t o = (int32_t)__shfl_up(end, (unsigned)d, kWave);
+        if (l >= d) end += o;
+    }
+    const int32_t start = end - length;
+    const int32_t total = shfl(end, kWave - 1);
+    const bool has = length > 0;
+    const uint64_t hm = ballot(has);
+    if (has) {
+        lds(sh->seg)[rank_in(hm)].shift = begin - start;
+        lds(sh->seg)[rank_in(hm)].nd = nd_own;
+    }
+    int32_t hits = 0;
+    for (int32_t b = 0; b < total; b += kWindows * kWave) {
+        wave_sync();
+        if (l < 2 * kWindows) lds(sh->starts)[l] = 0u;
+        wave_sync();
+        if (has && start >= b && start - b < kWindows * kWave)
+            atomicOr(&sh->starts[(start - b) >> 5], 1u << ((start - b) & 31));
+        wave_sync();
+        int32_t before = popc(ballot(has && start < b));  // segments that start before the window
+        int32_t u[kWindows], nd[kWindows];
+#pragma unroll
+        for (int j = 0; j < kWindows; ++j) {
+            const uint64_t m = uniform((uint64_t)lds(sh->starts)[2 * j] | ((uint64_t)lds(sh->starts)[2 * j + 1] << 32));
+            const int32_t r = before + rank_in(m) + (int32_t)((m >> l) & 1ull) - 1;
+            before += popc(m);
+            const int32_t f = b + j * kWave + l;
+            const bool in = f < total;
+            const int32_t shift = lds(sh->seg)[in ? r : 0].shift;
+            nd[j] = lds(sh->seg)[in ? r : 0].nd;
+            u[j] = in ? g.col[f + shift] : -1;
+        }
         bool bad = false;
 #pragma unroll
-        for (int j = 0; j < kChunkEdges; ++j) {
+        for (int j = 0; j < kWindows; ++j) {
             if (u[j] >= g.nv || u[j] < -1) {
                 bad = true;
                 u[j] = -1;
             }
         }
-        if (bad) {
-            GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, -1, g.nv);
+        if (ballot(bad)) {
+            if (bad) GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, -1, g.nv);
             break;
         }
-        int32_t old[kChunkEdges];
+        int32_t old[kWindows];
 #pragma unroll
-        for (int j = 0; j < kChunkEdges; ++j) old[j] = (u[j] >= 0) ? g.depth[u[j]] : 0;
+        for (int j = 0; j < kWindows; ++j) old[j] = u[j] >= 0 ? g.depth[u[j]] : 0;
 #pragma unroll
-        for (int j = 0; j < kChunkEdges; ++j) {
-            if (u[j] >= 0 && old[j] > nd)
-                old[j] = __hip_atomic_fetch_min(g.depth + u[j], nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else
-                old[j] = 0;
+        for (int j = 0; j < kWindows; ++j) {
+            if (old[j] > nd[j])
+                old[j] = __hip_atomic_fetch_min(g.depth + u[j], nd[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        // one spawn site for the improved vertices of the chunk (keeps the register count of the
-        // spawn path single)
-        uint32_t hits = 0;
 #pragma unroll
-        for (int j = 0; j < kChunkEdges; ++j) hits |= (old[j] > nd ? 1u : 0u) << j;
-        while (hits) {
-            const int j = __builtin_ctz(hits);
-            hits &= hits - 1u;
-            int32_t uj = u[0];
-#pragma unroll
-            for (int k = 1; k < kChunkEdges; ++k) uj = (j == k) ? u[k] : uj;
-            const int32_t us = g.row[uj];
-            const int32_t ue = g.row[uj + 1];
-            if (us < 0 || ue < us || (int64_t)ue > g.ne) {  // malformed offsets: never read past col
-                GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, uj, g.nv);
-                continue;
+        for (int j = 0; j < kWindows; ++j) {
+            const bool hit = old[j] > nd[j];
+            const uint64_t m = ballot(hit);
+            if (m == 0) continue;
+            if (hits + popc(m) > kHits) {
+                spawn_hits<NQ>(t, g, sh, hits);
+                hits = 0;
             }
-            __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(ue - us), BfsArg{uj, us, ue, nd});
+            if (hit) {
+                lds(sh->hit)[hits + rank_in(m)].u = u[j];
+                lds(sh->hit)[hits + rank_in(m)].nd = nd[j];
+            }
+            hits += popc(m);
+        }
+    }
+    if (hits) spawn_hits<NQ>(t, g, sh, hits);
+}
+
+template <int NQ>
+template <class L>
+__device__ __forceinline__ void Program<NQ>::run(L& lane) {
+    const BfsArgs& g = *lane.args;
+    const int32_t v = lane.template arg<int32_t>(0);
+    const int32_t s = lane.template arg<int32_t>(4);
+    const int32_t e = lane.template arg<int32_t>(8);
+    const int32_t d = lane.template arg<int32_t>(12);
+    // stale: v was reached by a shorter path meanwhile
+    if (ld32(reinterpret_cast<const int32_t*>(g.depth) + v) >= d) {
+        if (e - s > g.split) {
+            // up to kSplitFanout near-equal pieces, each routed by its own length
+            const int64_t len = (int64_t)e - s;
+            int32_t k = (int32_t)((len + g.split - 1) / g.split);
+            if (k > kSplitFanout) k = kSplitFanout;
+            for (int32_t i = 0; i < k; ++i) {
+                const int32_t ps = s + (int32_t)(len * i / k);
+                const int32_t pe = s + (int32_t)(len * (i + 1) / k);
+                __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
+            }
+        } else {
+            lane.coop = true;  // its edges: run_coop
         }
     }
     __gtap_finish_task(lane);
@@ -180,8 +262,10 @@ __device__ __forceinline__ void bfs_task(L& lane) {
 
 template <int NQ>
 template <class L>
-__device__ __forceinline__ void Program<NQ>::run(L& lane) {
-    bfs_task<NQ>(lane);
+__device__ __forceinline__ void Program<NQ>::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
+    (void)mask;
+    const int32_t s = (int32_t)lane.frame[1], e = (int32_t)lane.frame[2];
+    expand<NQ>(lane, *lane.args, sh, s, lane.coop ? e - s : 0, (int32_t)lane.frame[3] + 1);
 }
 
 // The wave form of the same task (queue 3 with 4 queues): all 64 lanes enter with one (v, s, e, d).
@@ -219,55 +303,7 @@ __device__ __forceinline__ void Program<NQ>::run_wave(W& wt) {
         wt.finish();
         return;
     }
-    const int32_t nd = d + 1;
-    const int32_t l = wt.lane;
-    for (int32_t b = s; b < e; b += kWave * kWaveChunk) {
-        int32_t u[kWaveChunk];
-#pragma unroll
-        for (int j = 0; j < kWaveChunk; ++j) {
-            const int32_t i = b + j * kWave + l;
-            u[j] = (i < e) ? g.col[i] : -1;
-        }
-        bool bad = false;
-#pragma unroll
-        for (int j = 0; j < kWaveChunk; ++j) {
-            if (u[j] >= g.nv || u[j] < -1) {
-                bad = true;
-                u[j] = -1;
-            }
-        }
-        if (ballot(bad)) {
-            if (bad) GTAP_DEVICE_ERROR(*wt.dev, GTAP_ERROR_INVALID_ARGUMENT, wt.tid, -1, -1, g.nv);
-            break;
-        }
-        int32_t old[kWaveChunk];
-#pragma unroll
-        for (int j = 0; j < kWaveChunk; ++j) old[j] = (u[j] >= 0) ? g.depth[u[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < kWaveChunk; ++j) {
-            if (u[j] >= 0 && old[j] > nd)
-                old[j] = __hip_atomic_fetch_min(g.depth + u[j], nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else
-                old[j] = 0;
-        }
-        uint32_t hits = 0;
-#pragma unroll
-        for (int j = 0; j < kWaveChunk; ++j) hits |= (old[j] > nd ? 1u : 0u) << j;
-        while (hits) {
-            const int j = __builtin_ctz(hits);
-            hits &= hits - 1u;
-            int32_t uj = u[0];
-#pragma unroll
-            for (int k = 1; k < kWaveChunk; ++k) uj = (j == k) ? u[k] : uj;
-            const int32_t us = g.row[uj];
-            const int32_t ue = g.row[uj + 1];
-            if (us < 0 || ue < us || (int64_t)ue > g.ne) {
-                GTAP_DEVICE_ERROR(*wt.dev, GTAP_ERROR_INVALID_ARGUMENT, wt.tid, -1, uj, g.nv);
-                continue;
-            }
-            wt.spawn_detached_lane(F_BFS, route<NQ>(ue - us), BfsArg{uj, us, ue, nd});
-        }
-    }
+    expand<NQ>(wt, g, wt.sh, s, wt.lane == 0 ? e - s : 0, d + 1);
     wt.finish();
 }
 
@@ -335,6 +371,8 @@ using Bfs4 = gtap::bfs::Program<4>;
 
 namespace {
 
+constexpr int32_t kMaxSplit = 1 << 20;   // 64 ranges of a round stay within 32-bit edge counts
+
 __global__ void bfs_init_depth(int32_t* depth, int32_t nv, int32_t source) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -354,6 +392,7 @@ extern "C" int gtap_bfs(const int32_t* row, const int32_t* col, int32_t nv, int6
         return host::invalid_argument("gtap_bfs: bad graph arguments");
     if (num_queues != 1 && num_queues != 4) return host::invalid_argument("gtap_bfs: num_queues must be 1 or 4");
     if (split <= 0) split = 64;
+    if (split > kMaxSplit) split = kMaxSplit;
     host::Runtime& R = host::rt();
     if (!R.initialized) {
         int st = gtap_initialize();

@@ -126,6 +126,26 @@ def test_bfs_bad_column_in_a_hub_is_reported(queues):
     assert st["error_code"] == 0 and np.array_equal(depth, oracle.bfs(row, col, 0))
 
 
+@pytest.mark.parametrize("degrees", [[1] * 200, [63] * 70, [64] * 70, [65] * 70, [0, 7, 0, 64, 1, 0, 511, 3] * 30,
+                                     [512, 0, 1] * 20, [200] * 64])
+@pytest.mark.parametrize("queues,split", [(1, 64), (1, 7), (4, 64), (1, 1 << 30), (4, 600)])
+def test_bfs_flat_edge_windows(degrees, queues, split):
+    """The ranges of a round are scanned as one sequence of 64-edge windows: ranges that start
+    and end at and around window and step borders, empty ranges between them, and more
+    improved vertices than the hit list holds."""
+    print(f"case bfs windows degrees={degrees[:8]} queues={queues} split={split}", flush=True)
+    k = len(degrees)
+    rng = np.random.default_rng(k + split % 1000)
+    n = 1 + k + 3000
+    adj = [np.arange(1, k + 1)] + [rng.integers(0, n, d) for d in degrees]
+    adj += [rng.integers(0, n, rng.integers(0, 3)) for _ in range(n - 1 - k)]
+    row = np.concatenate([[0], np.cumsum([len(a) for a in adj])]).astype(np.int32)
+    col = np.concatenate(adj).astype(np.int32)
+    depth, st = gtap_amd.bfs(row, col, 0, num_queues=queues, split=split)
+    assert st["error_code"] == 0
+    assert np.array_equal(depth, oracle.bfs(row, col, 0))
+
+
 def test_bfs_split_thresholds_agree():
     row, col = oracle.rmat_csr(13, 16, 11)
     ref = oracle.bfs(row, col, 0)
