@@ -68,6 +68,16 @@ template <class P>
 struct HasCoop<P, decltype((void)P::kCoop)> {
     static constexpr bool value = P::kCoop;
 };
+template <class P, class = void>
+struct WaveSharedOf {
+    struct type {
+        uint32_t unused;
+    };
+};
+template <class P>
+struct WaveSharedOf<P, decltype((void)sizeof(typename P::WaveShared))> {
+    using type = typename P::WaveShared;
+};
 
 // A program may count something over the whole launch (P::kLaneSum): each lane's run() adds to
 // lane.total, and the sums leave with the wave's statistics (ST_PROGRAM), which the summary
@@ -789,6 +799,7 @@ struct Lane {
     bool sum_join;          // the pending taskwait is an additive join
     uint32_t total;         // this lane's part of the launch's count (HasLaneSum programs)
     bool coop;              // run_coop finishes this task's body (HasCoop programs)
+    uint32_t coop_arg;      // what the body leaves for run_coop
     int64_t jsum;           // sum of the children's results, after an additive join
     uint64_t join_delta;    // what finishing adds to the parent's join word
     uint32_t frame[FW];     // the first frame words, loaded when the round starts
@@ -913,6 +924,11 @@ struct Lane {
         return true;
     }
 
+    // `count` children that run_coop will spawn with spawn_round: they count as spawned here.
+    __device__ __forceinline__ void will_spawn_sum(uint32_t count) {
+        child_sum += count;
+        child_count += count;
+    }
     // taskwait over children spawned with spawn_sum: when the task resumes at `next_state`,
     // join_sum() is the sum of their results (0 when there were none). Every child joined
     // here must be a spawn_sum child.
@@ -1090,6 +1106,93 @@ __device__ __forceinline__ uint32_t run_wave_task(const GtapDev& dev, const type
         (void)dev; (void)args; (void)w; (void)wave_shared; (void)me; (void)tid;
         parent_out = kNoParent;
         return OUT_FINISHED;
+    }
+}
+
+// ------------------------------------------------------------------ spawns of a whole round
+// Spawns the children of a round's tasks together, from run_coop: lane l's task (func, tid) gets
+// `count` children of an additive join on lane queue QQ, the i-th with arguments next(i). All
+// lanes take part, so the id stack's top, the queue's tail and its window masks are wave-uniform
+// and stay in scalar registers from one child index to the next. Spawning inside run(), where
+// only some lanes are active, reads and writes them in LDS for every child, a chain of about 600
+// cycles each: a round of n-queens(14) spent 2.1 us in task bodies that way, and 1.3 us this way.
+template <class P, int QQ, typename A, class Next>
+__device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next next) {
+    static_assert(sizeof(A) % 8 == 0 && sizeof(A) / 4 <= P::kFrameWords, "arguments must fit the loaded frame");
+    static_assert(QQ < CtxShape<P>::kQL, "a lane queue");
+    const GtapDev& dev = *L.dev;
+    WaveCtxOf<P>* w = L.w;
+    const int lane = lane_id();
+    uint32_t top = uniform(vld(&w->free_top));
+    uint32_t t = uniform(vld(&w->tail[QQ]));
+    uint32_t dtop = uniform(vld(&w->top_cache[QQ]));
+    uint64_t vmask = uniform(vld(&w->valid[QQ]));
+    uint64_t lmask = uniform(vld(&w->inlds[QQ]));
+    const uint32_t nstage0 = uniform(vld(&w->nstage));
+    uint32_t nstage = nstage0, spawned = 0, evicted = 0;
+    for (uint32_t i = 0;; ++i) {
+        const bool has = count > i;
+        const uint64_t m = ballot(has);
+        if (m == 0) break;
+        const uint32_t cnt = (uint32_t)popc(m), r = (uint32_t)rank_in(m);
+        if (top < cnt) {
+            if (lane == 0) vst(&w->free_top, top);
+            while (top < kRefillTarget) {
+                refill_chunk(dev, w, L.me, (kRefillTarget - top + kChunk - 1) / kChunk);
+                top = uniform(vld(&w->free_top));
+            }
+        }
+        if (t + cnt - dtop > dev.cap - kMargin) dtop = uniform((uint32_t)(ld64(dq_word_ptr(dev, QQ, L.me)) >> 32));
+        if (t + cnt - dtop > dev.cap - kMargin) {
+            if (lane == 0) GTAP_DEVICE_ERROR(dev, GTAP_ERROR_QUEUE_OVERFLOW, L.tid, QQ, t + cnt - dtop, dev.cap - kMargin);
+            break;
+        }
+        const uint32_t pos = t + r, slot = pos & (kWave - 1);
+        const bool spill = has && ((vmask >> slot) & 1ull);  // the slot's entry, at pos - 64, is pushed out
+        if (ballot(spill)) {
+            const bool rec = spill && ((lmask >> slot) & 1ull);
+            const uint64_t om = ballot(rec);
+            const uint32_t on = (uint32_t)popc(om);
+            const bool staged = nstage + on <= CtxShape<P>::kEvictStage;
+            if (spill) {
+                const uint32_t oid = vld(&w->mirror[QQ][slot]);
+                if (rec) {
+                    const uint32_t* d = &w->desc[QQ][slot][0];
+                    if (staged) stage_from_desc<P>(w, nstage + (uint32_t)rank_in(om), oid, d);
+                    else record_from_desc<P>(dev, L.rs, oid, d);
+                }
+                st32(dq_slot_ptr(dev, QQ, L.me, pos - kWave), oid);
+            }
+            if (staged) nstage += on;
+            evicted += on;
+        }
+        if (has) {
+            const A a = next(i);
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
+            vst(&w->mirror[QQ][slot], vld(&w->free_ids[top - 1 - r]));
+            uint32_t* d = &w->desc[QQ][slot][0];
+            vst(&d[0], hdr_word0(L.func, 0, QQ));
+            vst(&d[1], L.tid);
+            vst(&d[2], kResSum);
+#pragma unroll
+            for (int k = 0; k < (int)(sizeof(A) / 4); ++k) vst(&d[3 + k], src[k]);
+        }
+        const uint64_t range = rotl64(low_bits(cnt), t);
+        vmask |= range;
+        lmask |= range;
+        t += cnt;
+        top -= cnt;
+        spawned += cnt;
+    }
+    if (lane == 0) {
+        vst(&w->free_top, top);
+        vst(&w->tail[QQ], t);
+        vst(&w->top_cache[QQ], dtop);
+        vst(&w->valid[QQ], vmask);
+        vst(&w->inlds[QQ], lmask);
+        if (nstage != nstage0) vst(&w->nstage, nstage);
+        vst(&w->spawns, vld(&w->spawns) + spawned);
+        if (evicted) vst(&w->overflowed, vld(&w->overflowed) + evicted);
     }
 }
 
@@ -1868,7 +1971,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         }
         if constexpr (HasCoop<P>::value) {
             const uint64_t cm = ballot(L.coop);
-            if (cm) P::run_coop(L, cm, reinterpret_cast<typename P::WaveShared*>(wave_shared));
+            if (cm) P::run_coop(L, cm, reinterpret_cast<typename WaveSharedOf<P>::type*>(wave_shared));
         }
         phase_mark(PH_RUN);
 
@@ -2137,17 +2240,6 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
 }
 
 // Launch shape: 256-thread workgroups (4 waves), one WaveCtx per wave in LDS.
-template <class P, class = void>
-struct WaveSharedOf {
-    struct type {
-        uint32_t unused;
-    };
-};
-template <class P>
-struct WaveSharedOf<P, decltype((void)sizeof(typename P::WaveShared))> {
-    using type = typename P::WaveShared;
-};
-
 template <class P, int Sched = kSchedWS, bool Prof = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WavesPerSimd<P>::value)))
 void thread_kernel(GtapDev dev, typename P::Args args) {

@@ -51,6 +51,7 @@ struct ProgramT {
     static constexpr int kQueues = 1;
     // the default form is also built with the global-queue and Chase-Lev schedulers
     static constexpr bool kSchedVariants = kSum;
+    static constexpr bool kCoop = kSum;  // a round's children are spawned by run_coop
     static constexpr int kWavesPerSimd = kSum ? 4 : 1;
     static constexpr int kFrameWords = kSum ? 4 : 6;  // row, cols, diag, anti (, k, pad)
     static constexpr uint32_t kMaxFunc = F_NQ;
@@ -60,6 +61,8 @@ struct ProgramT {
     };
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
+    template <class L, class S>
+    __device__ __forceinline__ static void run_coop(L& lane, uint64_t mask, S* sh);
 };
 using Program = ProgramT<true>;
 using SlotProgram = ProgramT<false>;
@@ -80,13 +83,19 @@ __device__ __forceinline__ void nq_task(L& lane) {
             const uint32_t mask = (N < 32) ? ((1u << N) - 1u) : 0xFFFFFFFFu;
             uint32_t avail = mask & ~(cols | diag | anti);
             int32_t k = 0;
-            while (avail) {
-                const uint32_t p = avail & (0u - avail);
-                avail -= p;
-                const NqArg child{row + 1, cols | p, (diag | p) << 1, (anti | p) >> 1};
-                if constexpr (kSum) __gtap_spawn_task_sum(lane, F_NQ, 0, child);
-                else __gtap_spawn_task(lane, F_NQ, 0, kOffCounts + 8 * k, child);
-                ++k;
+            if constexpr (kSum) {
+                k = popc32(avail);
+                lane.coop = k != 0;  // the children: run_coop
+                lane.coop_arg = avail;
+                lane.will_spawn_sum((uint32_t)k);
+            } else {
+                while (avail) {
+                    const uint32_t p = avail & (0u - avail);
+                    avail -= p;
+                    const NqArg child{row + 1, cols | p, (diag | p) << 1, (anti | p) >> 1};
+                    __gtap_spawn_task(lane, F_NQ, 0, kOffCounts + 8 * k, child);
+                    ++k;
+                }
             }
             if (k == 0) {  // dead end: no legal column in this row
                 __gtap_return(lane, (int64_t)0);
@@ -126,6 +135,22 @@ template <bool kSum>
 template <class L>
 __device__ __forceinline__ void ProgramT<kSum>::run(L& lane) {
     nq_task<kSum>(lane);
+}
+
+// One child per free column of the task's row, lowest first.
+template <bool kSum>
+template <class L, class S>
+__device__ __forceinline__ void ProgramT<kSum>::run_coop(L& lane, uint64_t mask, S* sh) {
+    (void)mask;
+    (void)sh;
+    uint32_t avail = lane.coop ? lane.coop_arg : 0u;
+    const int32_t row = (int32_t)lane.frame[0];
+    const uint32_t cols = lane.frame[1], diag = lane.frame[2], anti = lane.frame[3];
+    spawn_round<ProgramT<kSum>, 0, NqArg>(lane, (uint32_t)popc32(avail), [&](uint32_t) {
+        const uint32_t p = avail & (0u - avail);
+        avail -= p;
+        return NqArg{row + 1, cols | p, (diag | p) << 1, (anti | p) >> 1};
+    });
 }
 
 }  // namespace nq
