@@ -1505,13 +1505,12 @@ __device__ __forceinline__ uint32_t try_steal(const GtapDev& dev, uint32_t me, u
 // expects, and reads its slots, which only it writes, while the CAS is under way: one round trip
 // where a load of the word, the CAS and the slot loads took three. A theft since the last look
 // makes the CAS fail and return the word.
+// `b` is the published bottom and `t` a lower bound of the top; both are brought up to date.
 template <class P>
-__device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, WaveCtxOf<P>* w, uint32_t me, uint32_t q,
-                                            uint32_t& tid_out, uint32_t max_items = kWave) {
+__device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, uint32_t me, uint32_t q, uint32_t& tid_out,
+                                            uint32_t max_items, uint32_t& b, uint32_t& t) {
     const int lane = lane_id();
     uint64_t* wp = dq_word_ptr(dev, q, me);
-    const uint32_t b = uniform(vld(&w->bottom[q]));
-    uint32_t t = uniform(vld(&w->top_cache[q]));
     uint32_t cap = ((int)q == HasWaveQueue<P>::value) ? 1u : (uint32_t)kWave;
     if (cap > max_items) cap = max_items;
     uint32_t k0 = 0;   // the number of slots read: positions [b - k0, b)
@@ -1521,10 +1520,7 @@ __device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, WaveCtxOf<P>* w,
     // (idle waves do not pop again, and quiescence may count them idle).
     while (true) {
         const int32_t sz = (int32_t)(b - t);
-        if (sz <= 0) {
-            if (lane == 0) vst(&w->top_cache[q], t);
-            return 0;
-        }
+        if (sz <= 0) return 0;
         const uint32_t k = (uint32_t)sz < cap ? (uint32_t)sz : cap;
         if (k0 == 0) {
             k0 = k;
@@ -1533,19 +1529,30 @@ __device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, WaveCtxOf<P>* w,
         uint64_t seen = ((uint64_t)t << 32) | (uint64_t)b;
         int ok = 0;
         if (lane == 0) ok = atomic_cas(wp, seen, ((uint64_t)t << 32) | (uint64_t)(b - k)) ? 1 : 0;
-        ok = shfl((int32_t)ok, 0);
+        ok = (int)uniform((uint32_t)ok);
         if (ok) {
             if (k != k0) tid = shfl(tid, lane + (int)(k0 - k));  // fewer than read: the newest k
             tid_out = tid;
-            if (lane == 0) {
-                vst(&w->bottom[q], b - k);
-                vst(&w->tail[q], b - k);
-                vst(&w->top_cache[q], t);
-            }
+            b -= k;
             return k;
         }
-        t = (uint32_t)(shfl(seen, 0) >> 32);
+        t = (uint32_t)(uniform(seen) >> 32);
     }
+}
+// The same on the wave's state in LDS, for a queue without private entries.
+template <class P>
+__device__ __forceinline__ uint32_t try_pop(const GtapDev& dev, WaveCtxOf<P>* w, uint32_t me, uint32_t q,
+                                            uint32_t& tid_out, uint32_t max_items = kWave) {
+    uint32_t b = vld(&w->bottom[q]), t = vld(&w->top_cache[q]);
+    b = uniform(b);
+    t = uniform(t);
+    const uint32_t k = try_pop<P>(dev, me, q, tid_out, max_items, b, t);
+    if (lane_id() == 0) {
+        if (k) vst(&w->tail[q], b);
+        vst(&w->bottom[q], b);
+        vst(&w->top_cache[q], t);
+    }
+    return k;
 }
 
 // ------------------------------------------------------------------ other schedulers
@@ -2030,11 +2037,34 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         }
         if (fin && fin_tid != 0u) free_id(dev, w, me, fin_tid);  // id 0 is the sink record
 
+        // The rest of the round works on register copies of the wave's queue state (positions,
+        // window masks), read from LDS once, together, and written back at the end: read where
+        // they are used they were a dozen LDS round trips in a row, about 0.5 us of a round.
+        uint32_t qt[Q], qb[Q], qc[Q];  // private tail, published bottom, lower bound of the top
+        uint64_t qv[Q], ql[Q];         // window masks: entries, entries held in LDS
+        uint32_t ns = vld(&w->nstage);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            qt[q] = vld(&w->tail[q]);
+            qb[q] = vld(&w->bottom[q]);
+            qc[q] = vld(&w->top_cache[q]);
+            qv[q] = vld(&w->valid[q]);
+            ql[q] = vld(&w->inlds[q]);
+        }
+        ns = uniform(ns);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            qt[q] = uniform(qt[q]);
+            qb[q] = uniform(qb[q]);
+            qc[q] = uniform(qc[q]);
+            qv[q] = uniform(qv[q]);
+            ql[q] = uniform(ql[q]);
+        }
         // choose the busiest queue, keep its newest <= 64 tasks, publish the rest
         uint32_t kmax = 0, cmax = 0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const uint32_t c = uniform(vld(&w->tail[q]) - vld(&w->bottom[q]));
+            const uint32_t c = qt[q] - qb[q];
             if (c > cmax) {
                 cmax = c;
                 kmax = (uint32_t)q;
@@ -2045,31 +2075,29 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         uint32_t next_tid = 0, next_slot = 0;
         bool next_lds = false;
         if (keep) {
-            const uint32_t t = uniform(vld(&w->tail[kmax]));
-            const uint64_t vmask = uniform(vld(&w->valid[kmax]));
-            const uint64_t lmask = uniform(vld(&w->inlds[kmax]));
-            if ((uint32_t)lane < keep) {
-                next_slot = (t - keep + (uint32_t)lane) & (kWave - 1);
-                next_tid = vld(&w->mirror[kmax][next_slot]);
-                next_lds = (lmask >> next_slot) & 1ull;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                if ((uint32_t)q == kmax) {
+                    const uint32_t t = qt[q];
+                    if ((uint32_t)lane < keep) {
+                        next_slot = (t - keep + (uint32_t)lane) & (kWave - 1);
+                        next_tid = vld(&w->mirror[q][next_slot]);
+                        next_lds = (ql[q] >> next_slot) & 1ull;
+                    }
+                    const uint64_t taken = rotl64(low_bits(keep), t - keep);
+                    qv[q] &= ~taken;
+                    ql[q] &= ~taken;
+                    qt[q] = t - keep;
+                }
             }
-            const uint64_t taken = rotl64(low_bits(keep), t - keep);
-            if (lane == 0) {
-                vst(&w->valid[kmax], vmask & ~taken);
-                vst(&w->inlds[kmax], lmask & ~taken);
-                vst(&w->tail[kmax], t - keep);
-                vst(&w->cur_queue, kmax);
-            }
+            if (lane == 0) vst(&w->cur_queue, kmax);
         }
         // records pushed out of the window by the continuations appended above
-        {
-            const uint32_t ns = uniform(vld(&w->nstage));
-            if (ns) {
-                wave_sync();
-                write_staged<P>(dev, L.rs, w, ns);
-                wave_sync();
-                if (lane == 0) vst(&w->nstage, 0u);
-            }
+        if (ns) {
+            wave_sync();
+            write_staged<P>(dev, L.rs, w, ns);
+            wave_sync();
+            if (lane == 0) vst(&w->nstage, 0u);
         }
         // write out what is published: entries still in the 64-slot window (lane i takes
         // slot i) get their deque slot, and their record if it is held in LDS
@@ -2080,16 +2108,14 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         uint32_t pub_to[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const uint32_t t = uniform(vld(&w->tail[q]));
-            const uint32_t b = uniform(vld(&w->bottom[q]));
+            const uint32_t t = qt[q];
+            const uint32_t b = qb[q];
             const bool retain = Sched != kSchedGQ && Q > 1 && q < QL && (uint32_t)q != kmax && !dev.epaq_publish;
             pub_to[q] = !retain ? t : ((int32_t)(t - b) > kWave ? t - kWave : b);
             if (retain && pub_to[q] != b) any_publish = true;
             if (!retain && t != b) {
                 any_publish = true;
-                const uint64_t vmask = uniform(vld(&w->valid[q]));
-                const uint64_t lmask = uniform(vld(&w->inlds[q]));
-                const bool mine = (vmask >> lane) & 1ull;
+                const bool mine = (qv[q] >> lane) & 1ull;
                 uint32_t oid = 0;
                 if (mine) {
                     const uint32_t pos = t - kWave + (((uint32_t)lane - t) & (kWave - 1));
@@ -2098,7 +2124,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                 }
                 if (q < QL) {
                     // records held in LDS: staged in record order, written together
-                    const bool stg = mine && ((lmask >> lane) & 1ull);
+                    const bool stg = mine && ((ql[q] >> lane) & 1ull);
                     const uint64_t sm = ballot(stg);
                     if (sm) {
                         if (stg) {
@@ -2119,42 +2145,38 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                         wave_sync();
                     }
                 }
-                if (lane == 0) {
-                    vst(&w->valid[q], (uint64_t)0);
-                    vst(&w->inlds[q], (uint64_t)0);
-                }
+                qv[q] = 0;
+                ql[q] = 0;
             }
         }
         if (any_publish) {
             complete_stores();  // records and slots of everything published below
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                const uint32_t b = uniform(vld(&w->bottom[q]));
+                const uint32_t b = qb[q];
                 const uint32_t t = pub_to[q];
                 if (t != b) {
                     if constexpr (Sched == kSchedGQ) {
                         gq_push<P>(dev, w, me, (uint32_t)q, b, t);
+                        qc[q] = t;
                     } else {
-                        // top_cache stays a lower bound of the top; the capacity check re-reads it
+                        // the top bound stays; the capacity check re-reads the word
                         if (lane == 0) atomic_add_noret(dq_word_ptr(dev, q, me), (uint64_t)(t - b));
                     }
-                    vst(&w->bottom[q], t);
+                    qb[q] = t;
                 }
             }
         }
         // a deque above half its capacity hands its oldest published tasks to the overflow ring
         if constexpr (Sched != kSchedGQ) {
             if (dev.ovf_cells != nullptr) {
-#pragma unroll 1
+#pragma unroll
                 for (int q = 0; q < Q; ++q) {
-                    const uint32_t b = uniform(vld(&w->bottom[q]));
-                    if (b - uniform(vld(&w->top_cache[q])) > dev.cap / 2) {
+                    if (qb[q] - qc[q] > dev.cap / 2) {
                         const uint64_t r = ovf_spill_deque(ovf_view(dev), (uint32_t)q, dq_word_ptr(dev, q, me),
                                                            dq_slot_ptr(dev, q, me, 0), dev.cap);
-                        if (lane == 0) {
-                            vst(&w->top_cache[q], (uint32_t)r);
-                            vst(&w->ring_spilled, vld(&w->ring_spilled) + (uint32_t)(r >> 32));
-                        }
+                        qc[q] = uniform((uint32_t)r);
+                        if (lane == 0) vst(&w->ring_spilled, vld(&w->ring_spilled) + (uint32_t)(r >> 32));
                     }
                 }
             }
@@ -2165,8 +2187,23 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         // wave runs dry. Their records are in HBM and load at the round's start.
         if constexpr (Sched == kSchedWS) {
             if (keep < bcap && (int)kmax != WQ) {
-                uint32_t ptid = 0;
-                const uint32_t k = try_pop<P>(dev, w, me, kmax, ptid, bcap - keep);
+                uint32_t ptid = 0, pb = qb[0], pc = qc[0];
+#pragma unroll
+                for (int q = 1; q < Q; ++q) {
+                    if ((uint32_t)q == kmax) {
+                        pb = qb[q];
+                        pc = qc[q];
+                    }
+                }
+                const uint32_t k = try_pop<P>(dev, me, kmax, ptid, bcap - keep, pb, pc);
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    if ((uint32_t)q == kmax) {
+                        if (k) qt[q] = pb;
+                        qb[q] = pb;
+                        qc[q] = pc;
+                    }
+                }
                 if (k) {
                     const int src = lane - (int)keep;
                     const uint32_t v = shfl(ptid, src < 0 ? 0 : src);
@@ -2178,6 +2215,16 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                     st.pops += 1;
                     if (lane == 0) vst(&w->cur_queue, kmax);
                 }
+            }
+        }
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                vst(&w->tail[q], qt[q]);
+                vst(&w->bottom[q], qb[q]);
+                vst(&w->top_cache[q], qc[q]);
+                vst(&w->valid[q], qv[q]);
+                vst(&w->inlds[q], ql[q]);
             }
         }
         phase_mark(PH_PUBLISH);
