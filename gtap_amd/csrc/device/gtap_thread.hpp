@@ -417,22 +417,6 @@ __device__ __forceinline__ uint32_t alloc_id(const GtapDev& dev, W* w, uint32_t 
     return id;
 }
 
-template <class W>
-__device__ __forceinline__ void free_id(const GtapDev& dev, W* w, uint32_t me, uint32_t id) {
-    const uint64_t m = active_mask();
-    const uint32_t cnt = (uint32_t)popc(m);
-    const uint32_t r = (uint32_t)rank_in(m);
-    uint32_t top = uniform(vld(&w->free_top));
-    if (top + cnt > kFreeCap) {
-        while (top > kSpillTarget) {
-            spill_chunk(dev, w, me);
-            top = uniform(vld(&w->free_top));
-        }
-    }
-    vst(&w->free_ids[top + r], id);
-    vst(&w->free_top, top + cnt);
-}
-
 // ------------------------------------------------------------------ deque append
 
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, uint32_t r) {
@@ -1109,6 +1093,51 @@ __device__ __forceinline__ uint32_t run_wave_task(const GtapDev& dev, const type
     }
 }
 
+// ------------------------------------------------------------------ appends by the whole wave
+// The lanes of `m` (`mine`) each append an entry with id `id` to the private end of queue q, whose
+// state the caller holds in registers: tail, lower bound of the deque's top, window masks, and
+// the number of records staged this round. All lanes call it. kDesc: the new entries are held in
+// LDS (the caller fills their descriptors), else their records are in HBM. As queue_append does, it
+// writes out the entries it pushes out of the 64-slot window and reports a full deque (nothing is
+// appended and nothing changes then).
+template <class P, bool kDesc>
+__device__ __forceinline__ bool window_append(const GtapDev& dev, WaveCtxOf<P>* w, __amdgpu_buffer_rsrc_t rs, uint32_t me,
+                                              int q, uint64_t m, bool mine, uint32_t id, uint32_t& tail, uint32_t& dtop,
+                                              uint64_t& vmask, uint64_t& lmask, uint32_t& nstage) {
+    constexpr int QL = CtxShape<P>::kQL;
+    const uint32_t cnt = (uint32_t)popc(m), r = (uint32_t)rank_in(m);
+    if (tail + cnt - dtop > dev.cap - kMargin) dtop = uniform((uint32_t)(ld64(dq_word_ptr(dev, q, me)) >> 32));
+    if (tail + cnt - dtop > dev.cap - kMargin) {
+        if (lane_id() == 0) GTAP_DEVICE_ERROR(dev, GTAP_ERROR_QUEUE_OVERFLOW, -1, q, tail + cnt - dtop, dev.cap - kMargin);
+        return false;
+    }
+    const uint32_t slot = (tail + r) & (kWave - 1);
+    const bool spill = mine && ((vmask >> slot) & 1ull);  // the slot's entry, 64 positions back, is pushed out
+    if (ballot(spill)) {
+        const bool rec = spill && q < QL && ((lmask >> slot) & 1ull);
+        const uint64_t om = ballot(rec);
+        const uint32_t on = (uint32_t)popc(om);
+        const bool staged = nstage + on <= CtxShape<P>::kEvictStage;
+        if (spill) {
+            const uint32_t oid = vld(&w->mirror[q][slot]);
+            if (rec) {
+                const uint32_t* d = &w->desc[q < QL ? q : 0][slot][0];
+                if (staged) stage_from_desc<P>(w, nstage + (uint32_t)rank_in(om), oid, d);
+                else record_from_desc<P>(dev, rs, oid, d);
+            }
+            st32(dq_slot_ptr(dev, q, me, tail + r - kWave), oid);
+        }
+        if (staged) nstage += on;
+        if (on && lane_id() == 0) vst(&w->overflowed, vld(&w->overflowed) + on);
+    }
+    if (mine) vst(&w->mirror[q][slot], id);
+    const uint64_t range = rotl64(low_bits(cnt), tail);
+    vmask |= range;
+    lmask = kDesc ? lmask | range : lmask & ~range;
+    tail += cnt;
+    return true;
+}
+
 // ------------------------------------------------------------------ spawns of a whole round
 // Spawns the children of a round's tasks together, from run_coop: lane l's task (func, tid) gets
 // `count` children of an additive join on lane queue QQ, the i-th with arguments next(i). All
@@ -1129,7 +1158,7 @@ __device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next nex
     uint64_t vmask = uniform(vld(&w->valid[QQ]));
     uint64_t lmask = uniform(vld(&w->inlds[QQ]));
     const uint32_t nstage0 = uniform(vld(&w->nstage));
-    uint32_t nstage = nstage0, spawned = 0, evicted = 0;
+    uint32_t nstage = nstage0, spawned = 0;
     for (uint32_t i = 0;; ++i) {
         const bool has = count > i;
         const uint64_t m = ballot(has);
@@ -1142,45 +1171,19 @@ __device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next nex
                 top = uniform(vld(&w->free_top));
             }
         }
-        if (t + cnt - dtop > dev.cap - kMargin) dtop = uniform((uint32_t)(ld64(dq_word_ptr(dev, QQ, L.me)) >> 32));
-        if (t + cnt - dtop > dev.cap - kMargin) {
-            if (lane == 0) GTAP_DEVICE_ERROR(dev, GTAP_ERROR_QUEUE_OVERFLOW, L.tid, QQ, t + cnt - dtop, dev.cap - kMargin);
-            break;
-        }
-        const uint32_t pos = t + r, slot = pos & (kWave - 1);
-        const bool spill = has && ((vmask >> slot) & 1ull);  // the slot's entry, at pos - 64, is pushed out
-        if (ballot(spill)) {
-            const bool rec = spill && ((lmask >> slot) & 1ull);
-            const uint64_t om = ballot(rec);
-            const uint32_t on = (uint32_t)popc(om);
-            const bool staged = nstage + on <= CtxShape<P>::kEvictStage;
-            if (spill) {
-                const uint32_t oid = vld(&w->mirror[QQ][slot]);
-                if (rec) {
-                    const uint32_t* d = &w->desc[QQ][slot][0];
-                    if (staged) stage_from_desc<P>(w, nstage + (uint32_t)rank_in(om), oid, d);
-                    else record_from_desc<P>(dev, L.rs, oid, d);
-                }
-                st32(dq_slot_ptr(dev, QQ, L.me, pos - kWave), oid);
-            }
-            if (staged) nstage += on;
-            evicted += on;
-        }
+        const uint32_t id = has ? vld(&w->free_ids[top - 1 - r]) : 0u;
+        const uint32_t t0 = t;
+        if (!window_append<P, true>(dev, w, L.rs, L.me, QQ, m, has, id, t, dtop, vmask, lmask, nstage)) break;
         if (has) {
             const A a = next(i);
             const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
-            vst(&w->mirror[QQ][slot], vld(&w->free_ids[top - 1 - r]));
-            uint32_t* d = &w->desc[QQ][slot][0];
+            uint32_t* d = &w->desc[QQ][(t0 + r) & (kWave - 1)][0];
             vst(&d[0], hdr_word0(L.func, 0, QQ));
             vst(&d[1], L.tid);
             vst(&d[2], kResSum);
 #pragma unroll
             for (int k = 0; k < (int)(sizeof(A) / 4); ++k) vst(&d[3 + k], src[k]);
         }
-        const uint64_t range = rotl64(low_bits(cnt), t);
-        vmask |= range;
-        lmask |= range;
-        t += cnt;
         top -= cnt;
         spawned += cnt;
     }
@@ -1192,7 +1195,6 @@ __device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next nex
         vst(&w->inlds[QQ], lmask);
         if (nstage != nstage0) vst(&w->nstage, nstage);
         vst(&w->spawns, vld(&w->spawns) + spawned);
-        if (evicted) vst(&w->overflowed, vld(&w->overflowed) + evicted);
     }
 }
 
@@ -2015,9 +2017,50 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         complete_stores();  // results, suspended records and child records of this round
         phase_mark(PH_WAIT);
         uint32_t ready = kNoParent, ready_q = 0;
-        if (fin && fin_parent != kNoParent) {
-            // the parent's join word: the last child also reads the resume queue
-            const uint64_t old = atomic_add(reinterpret_cast<uint64_t*>(rec_ptr(dev, fin_parent) + kHdrJoin), fin_delta);
+        const bool joins = fin && fin_parent != kNoParent;
+        uint64_t old = 0;
+        // the parent's join word: the last child also reads the resume queue
+        if (joins) old = atomic_add(reinterpret_cast<uint64_t*>(rec_ptr(dev, fin_parent) + kHdrJoin), fin_delta);
+        // The rest of the round works on register copies of the wave's queue state (positions,
+        // window masks, the id stack's top), read from LDS once, together, while the join
+        // atomics are under way, and written back at the end: read where they are used they were
+        // some twenty LDS round trips in a row, nearly 1 us of a round.
+        uint32_t qt[Q], qb[Q], qc[Q];  // private tail, published bottom, lower bound of the top
+        uint64_t qv[Q], ql[Q];         // window masks: entries, entries held in LDS
+        uint32_t ftop = vld(&w->free_top);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            qt[q] = vld(&w->tail[q]);
+            qb[q] = vld(&w->bottom[q]);
+            qc[q] = vld(&w->top_cache[q]);
+            qv[q] = vld(&w->valid[q]);
+            ql[q] = vld(&w->inlds[q]);
+        }
+        ftop = uniform(ftop);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            qt[q] = uniform(qt[q]);
+            qb[q] = uniform(qb[q]);
+            qc[q] = uniform(qc[q]);
+            qv[q] = uniform(qv[q]);
+            ql[q] = uniform(ql[q]);
+        }
+        // the finished tasks' ids (id 0 is the sink record)
+        {
+            const bool frees = fin && fin_tid != 0u;
+            const uint64_t m = ballot(frees);
+            const uint32_t cnt = (uint32_t)popc(m);
+            if (ftop + cnt > kFreeCap) {
+                if (lane == 0) vst(&w->free_top, ftop);
+                while (ftop > kSpillTarget) {
+                    spill_chunk(dev, w, me);
+                    ftop = uniform(vld(&w->free_top));
+                }
+            }
+            if (frees) vst(&w->free_ids[ftop + (uint32_t)rank_in(m)], fin_tid);
+            ftop += cnt;
+        }
+        if (joins) {
             const uint32_t left = fin_sum ? (uint32_t)old & kSumMaxCount : (uint32_t)old;
             if (left == 1u) {
                 ready = fin_parent;
@@ -2030,35 +2073,18 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
             __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the join atomics have returned
             phase_mark(PH_JOIN);
         }
+        uint32_t ns = 0;  // records staged for the writes below: entries the continuations push out
         if (ballot(ready != kNoParent)) {
             if (ready != kNoParent && ready >= dev.nrecs) complete_job<P>(dev, ready);
-            if (ready != kNoParent && ready < dev.nrecs)
-                queue_append<P, false>(dev, w, me, ready_q < (uint32_t)Q ? ready_q : 0u, ready, nullptr);
-        }
-        if (fin && fin_tid != 0u) free_id(dev, w, me, fin_tid);  // id 0 is the sink record
-
-        // The rest of the round works on register copies of the wave's queue state (positions,
-        // window masks), read from LDS once, together, and written back at the end: read where
-        // they are used they were a dozen LDS round trips in a row, about 0.5 us of a round.
-        uint32_t qt[Q], qb[Q], qc[Q];  // private tail, published bottom, lower bound of the top
-        uint64_t qv[Q], ql[Q];         // window masks: entries, entries held in LDS
-        uint32_t ns = vld(&w->nstage);
+            const bool resumes = ready != kNoParent && ready < dev.nrecs;
+            if (ready_q >= (uint32_t)Q) ready_q = 0u;
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            qt[q] = vld(&w->tail[q]);
-            qb[q] = vld(&w->bottom[q]);
-            qc[q] = vld(&w->top_cache[q]);
-            qv[q] = vld(&w->valid[q]);
-            ql[q] = vld(&w->inlds[q]);
-        }
-        ns = uniform(ns);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            qt[q] = uniform(qt[q]);
-            qb[q] = uniform(qb[q]);
-            qc[q] = uniform(qc[q]);
-            qv[q] = uniform(qv[q]);
-            ql[q] = uniform(ql[q]);
+            for (int q = 0; q < Q; ++q) {
+                const bool mine = resumes && ready_q == (uint32_t)q;
+                const uint64_t m = ballot(mine);
+                if (m == 0) continue;
+                (void)window_append<P, false>(dev, w, L.rs, me, q, m, mine, ready, qt[q], qc[q], qv[q], ql[q], ns);
+            }
         }
         // choose the busiest queue, keep its newest <= 64 tasks, publish the rest
         uint32_t kmax = 0, cmax = 0;
@@ -2097,7 +2123,6 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
             wave_sync();
             write_staged<P>(dev, L.rs, w, ns);
             wave_sync();
-            if (lane == 0) vst(&w->nstage, 0u);
         }
         // write out what is published: entries still in the 64-slot window (lane i takes
         // slot i) get their deque slot, and their record if it is held in LDS
@@ -2218,6 +2243,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
             }
         }
         if (lane == 0) {
+            vst(&w->free_top, ftop);
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
                 vst(&w->tail[q], qt[q]);
