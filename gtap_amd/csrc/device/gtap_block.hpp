@@ -645,6 +645,8 @@ __device__ void block_scheduler(const GtapDev& dev, const typename P::Args& args
         s[ST_STEAL_ATTEMPTS] = lp.attempts;
         s[ST_JOBS] = lp.jobs;
         s[ST_REFILLS] = c->refills;
+        s[ST_PUBLISHED] = s[ST_OVERFLOWED] = s[ST_SUSPENDED] = 0;
+        s[ST_RING_SPILLED] = s[ST_RING_TAKEN] = s[ST_PROGRAM] = 0;
         s[ST_START_TICKS] = lp.t_begin;
         s[ST_END_TICKS] = now_ticks();
     }

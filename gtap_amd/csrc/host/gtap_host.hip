@@ -159,8 +159,38 @@ GtapDev make_dev(uint32_t nworkers, uint32_t term_mode, uint32_t njobs, gtap_job
     return d;
 }
 
-// Clears the per-launch state: control words, deque words, id-pool ring, statistics.
-__global__ void reset_kernel(GtapDev dev, gtap_job job0, int32_t write_job0, int32_t arm) {
+// Frees what an aborted or first-task launch left in the rings, whose positions are never reset.
+// Overflow ring q: cells between the head and the tickets are freed for the next lap and the head
+// moves up to the tickets. Id ring s: the ids of its full cells are given up (every launch starts
+// with all ids fresh), each cell is freed for the next lap and the dequeue position moves up to the
+// enqueue position. One workgroup per ring, so the position moves after every cell is freed.
+__device__ __forceinline__ void drain_ovf_ring(const GtapDev& dev, uint32_t q) {
+    const uint64_t head = ld64(dev.ovf_ctl + (size_t)q * 32), tickets = ld64(dev.ovf_ctl + (size_t)q * 32 + 16);
+    for (uint64_t p = head + threadIdx.x; p < tickets; p += blockDim.x)
+        st64(dev.ovf_cells + (size_t)q * dev.ovf_cap + (p & (dev.ovf_cap - 1)), ((p + dev.ovf_cap) & 0x3FFFFFFFull) << 32);
+    __syncthreads();
+    if (threadIdx.x == 0 && head != tickets) st64(dev.ovf_ctl + (size_t)q * 32, tickets);
+}
+__device__ __forceinline__ void drain_id_ring(const GtapDev& dev, uint32_t s) {
+    uint32_t* enq = reinterpret_cast<uint32_t*>(dev.pool_ctl + (size_t)s * 32);
+    uint32_t* deq = reinterpret_cast<uint32_t*>(dev.pool_ctl + (size_t)s * 32 + 16);
+    const uint32_t d = ld32(deq), e = ld32(enq);
+    for (uint32_t i = threadIdx.x; i < e - d; i += blockDim.x)
+        st32(dev.pool_seq + (size_t)s * dev.ncells + ((d + i) & (dev.ncells - 1)), d + i + dev.ncells);
+    __syncthreads();
+    if (threadIdx.x == 0 && d != e) st32(deq, e);
+}
+
+// Clears the per-launch state: control words, deque words and what the rings hold, and (when an
+// entry kernel is armed, whose launch may run fewer workers than are provisioned) the statistics;
+// the workers of a launch write their whole rows. One kernel, one pass: a drain kernel of one
+// workgroup before it and a pass over all 16 MB of id-ring sequence numbers took 4 us each.
+__global__ void __launch_bounds__(256) reset_kernel(GtapDev dev, gtap_job job0, int32_t write_job0, int32_t arm) {
+    const uint32_t rings = (dev.ovf_cells ? dev.nqueues : 0u) + dev.nshards;
+    for (uint32_t r = blockIdx.x; r < rings; r += gridDim.x) {
+        if (r < dev.nshards) drain_id_ring(dev, r);
+        else drain_ovf_ring(dev, r - dev.nshards);
+    }
     const uint64_t gid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
     const uint64_t gs = (uint64_t)gridDim.x * blockDim.x;
     if (write_job0 && gid < sizeof(gtap_job) / 4)
@@ -173,9 +203,8 @@ __global__ void reset_kernel(GtapDev dev, gtap_job job0, int32_t write_job0, int
                          ? (int32_t)dev.static_jobs
                          : (i == CTL_ARMED * 32 ? arm : 0);
     for (uint64_t i = gid; i < (uint64_t)dev.nqueues * dev.nworkers; i += gs) dev.dq_word[i * 16] = 0;
-    for (uint64_t i = gid; i < (uint64_t)dev.nshards * dev.ncells; i += gs)
-        dev.pool_seq[i] = (uint32_t)(i & (dev.ncells - 1));
-    for (uint64_t i = gid; i < (uint64_t)dev.nworkers * ST_COUNT; i += gs) dev.stats[i] = 0;
+    if (arm)
+        for (uint64_t i = gid; i < (uint64_t)dev.nworkers * ST_COUNT; i += gs) dev.stats[i] = 0;
     if (dev.gq_ctl)
         for (uint64_t i = gid; i < (uint64_t)dev.nqueues * 3 * 16; i += gs) dev.gq_ctl[i] = 0;
     if (dev.prof_phase)
@@ -187,25 +216,9 @@ __global__ void reset_kernel(GtapDev dev, gtap_job job0, int32_t write_job0, int
             dev.prof_counts[i] = 0;
         }
     }
-    // ring positions start at 0; the fresh-id counter starts at 64 (ids 0..63 are
-    // reserved, id 0 is the sink record), above the workers' fixed first ranges
-    for (uint64_t i = gid; i < (uint64_t)dev.nshards * 32 + 32; i += gs)
-        dev.pool_ctl[i] = (i == (uint64_t)dev.nshards * 32) ? 64ull + (uint64_t)dev.nworkers * dev.static_ids : 0ull;
-}
-
-// The overflow rings keep their positions from launch to launch. A launch that ended early
-// (an error, first-task termination with detached tasks still queued) can leave tickets
-// between the head and the ticket counter: their cells are freed for the next lap and the
-// head moves up to the tickets. One workgroup, so the head moves after every cell is freed.
-__global__ void __launch_bounds__(256) ovf_drain_kernel(GtapDev dev) {
-    for (uint32_t q = 0; q < dev.nqueues; ++q) {
-        const uint64_t head = ld64(dev.ovf_ctl + (size_t)q * 32), tickets = ld64(dev.ovf_ctl + (size_t)q * 32 + 16);
-        for (uint64_t p = head + threadIdx.x; p < tickets; p += blockDim.x)
-            st64(dev.ovf_cells + (size_t)q * dev.ovf_cap + (p & (dev.ovf_cap - 1)), ((p + dev.ovf_cap) & 0x3FFFFFFFull) << 32);
-        __syncthreads();
-        if (threadIdx.x == 0) st64(dev.ovf_ctl + (size_t)q * 32, tickets);
-        __syncthreads();
-    }
+    // the fresh-id counter starts at 64 (ids 0..63 are reserved, id 0 is the sink record), above
+    // the workers' fixed first ranges
+    if (gid == 0) dev.pool_ctl[(uint64_t)dev.nshards * 32] = 64ull + (uint64_t)dev.nworkers * dev.static_ids;
 }
 
 // Every cell free for its first lap (the tag of cell i is i), positions at 0.
@@ -216,15 +229,19 @@ __global__ void ovf_init_kernel(uint64_t* cells, uint64_t* ctl, uint32_t nqueues
     for (uint64_t i = gid; i < (uint64_t)nqueues * 32; i += gs) ctl[i] = 0;
 }
 
+// The id rings' cells free for their first lap (cell i of a ring: sequence number i).
+__global__ void pool_init_kernel(uint32_t* seq, uint32_t nshards, uint32_t ncells) {
+    const uint64_t gid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    const uint64_t gs = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = gid; i < (uint64_t)nshards * ncells; i += gs) seq[i] = (uint32_t)(i & (ncells - 1));
+}
+
 int enqueue_reset(const GtapDev& dev, hipStream_t stream, const gtap_job* job0, bool arm) {
     gtap_job j;
     if (job0) j = *job0;
     else memset(&j, 0, sizeof(j));
-    if (dev.ovf_cells) {
-        hipLaunchKernelGGL(ovf_drain_kernel, dim3(1), dim3(256), 0, stream, dev);
-        GTAP_HIP_TRY(hipGetLastError());
-    }
-    hipLaunchKernelGGL(reset_kernel, dim3(1024), dim3(256), 0, stream, dev, j, job0 ? 1 : 0, arm ? 1 : 0);
+    const uint32_t grid = dev.prof_max ? 1024u : 128u;
+    hipLaunchKernelGGL(reset_kernel, dim3(grid), dim3(256), 0, stream, dev, j, job0 ? 1 : 0, arm ? 1 : 0);
     GTAP_HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -238,37 +255,42 @@ int reset_launch_state(const GtapDev& dev, hipStream_t stream, const gtap_job* j
 }
 
 // One workgroup: sums the per-worker statistics of the launch that just ended and writes
-// them, the first error code and (on request) job-table slot 0 to the pinned summary.
-constexpr int kSummaryThreads = 256;
+// them, the first error code and (on request) job-table slot 0 to the pinned summary. Thread t sums
+// column t % 16, so a wave reads whole lines, 8 rows in flight per thread (15 us for 4096
+// workers with 256 threads that each read whole rows, 64 lines per load).
+constexpr int kSummaryThreads = 1024;
 __global__ void __launch_bounds__(kSummaryThreads) summary_kernel(GtapDev dev, LaunchSummary* out, int32_t copy_job0) {
-    __shared__ uint64_t part[ST_COUNT][kSummaryThreads];
+    __shared__ uint64_t part[kSummaryThreads];
     const uint32_t t = threadIdx.x;
-    uint64_t acc[ST_COUNT];
+    const uint32_t n = dev.nworkers * ST_COUNT;
+    uint64_t acc = 0;
+    constexpr uint32_t kStep = kSummaryThreads, kFlight = 8;
+    uint32_t i = t;
+    for (; i + (kFlight - 1) * kStep < n; i += kFlight * kStep) {
+        uint64_t v[kFlight];
 #pragma unroll
-    for (int i = 0; i < ST_COUNT; ++i) acc[i] = 0;
-    for (uint32_t w = t; w < dev.nworkers; w += kSummaryThreads) {
+        for (uint32_t j = 0; j < kFlight; ++j) v[j] = dev.stats[i + j * kStep];
 #pragma unroll
-        for (int i = 0; i < ST_COUNT; ++i) acc[i] += dev.stats[(size_t)w * ST_COUNT + i];
+        for (uint32_t j = 0; j < kFlight; ++j) acc += v[j];
     }
-#pragma unroll
-    for (int i = 0; i < ST_COUNT; ++i) part[i][t] = acc[i];
+    for (; i < n; i += kStep) acc += dev.stats[i];
+    part[t] = acc;
     __syncthreads();
-    for (uint32_t h = kSummaryThreads / 2; h > 0; h >>= 1) {
-        if (t < h) {
+    if (t < ST_COUNT) {
+        uint64_t sum = 0;
 #pragma unroll
-            for (int i = 0; i < ST_COUNT; ++i) part[i][t] += part[i][t + h];
-        }
-        __syncthreads();
+        for (int k = 0; k < kSummaryThreads / ST_COUNT; ++k) sum += part[k * ST_COUNT + t];
+        out->sums[t] = sum;
     }
-    if (t < ST_COUNT) out->sums[t] = part[t][0];
-    if (t == 0) {
+    if (t == 64) {
         out->error_code = dev.ctl[CTL_ERROR * 32];
         out->admission_holds = dev.ctl[CTL_ADMIT_HOLDS * 32];
         out->has_job0 = copy_job0;
     }
-    if (copy_job0 && t < sizeof(gtap_job) / 4)
-        reinterpret_cast<uint32_t*>(&out->job0)[t] = reinterpret_cast<const uint32_t*>(dev.jobs)[t];
+    if (copy_job0 && t >= 128 && t - 128 < sizeof(gtap_job) / 4)
+        reinterpret_cast<uint32_t*>(&out->job0)[t - 128] = reinterpret_cast<const uint32_t*>(dev.jobs)[t - 128];
 }
+static_assert(kSummaryThreads % ST_COUNT == 0, "a thread sums one column");
 
 int enqueue_summary(const GtapDev& dev, hipStream_t stream, bool copy_job0) {
     Runtime& R = rt();
@@ -512,6 +534,8 @@ int gtap_initialize(void) {
     GTAP_HIP_TRY(hipMemset(R.ovf_epoch, 0, 64 * 32 * sizeof(uint32_t)));
     hipLaunchKernelGGL(ovf_init_kernel, dim3(1024), dim3(256), 0, R.stream, R.ovf_cells, R.ovf_ctl, R.nqueues,
                        R.ovf_cap);
+    GTAP_HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(pool_init_kernel, dim3(1024), dim3(256), 0, R.stream, R.pool_seq, R.nshards, R.ncells);
     GTAP_HIP_TRY(hipGetLastError());
 
     GTAP_HIP_TRY(hipMalloc(&R.ctl, (size_t)CTL_COUNT * 32 * sizeof(int32_t)));

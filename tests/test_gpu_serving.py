@@ -51,3 +51,38 @@ def test_admission_holds_jobs_back_and_results_stay_exact():
         assert np.all(lat_r > 0)
     finally:
         st.close()
+
+
+def test_id_rings_carry_over_launches():
+    """The id rings keep their positions from launch to launch; what a launch leaves in them is
+    given up by the next one's reset. Served runs on a small pool park few ids per wave and so
+    pass ids through the rings; their leftovers must not be handed out again in later launches
+    (a doubled id would break results), and a launch that ends in an error must not either."""
+    st = gtap_amd.Stream(seed=47, njobs=200)
+    try:
+        exp = expected(st)
+        for k in range(4):
+            print(f"case served, launch {k} on the same rings", flush=True)
+            res, _, _, stats = st.serve(rate=100_000.0, arrival_seed=k, max_live=256)
+            assert np.array_equal(res, exp) and stats["error_code"] == 0
+            v, s = gtap_amd.fib(22 + k)
+            assert v == oracle.fib(22 + k) and s["tasks_executed"] == 3 * oracle.fib(23 + k) - 2
+            keys = oracle.gen_keys_u32(50_001, k)
+            assert np.array_equal(gtap_amd.cilksort(keys)[0], np.sort(keys))
+            rp, ci, va = gtap_amd.spmv_random(50000, 4, 1)
+            with pytest.raises(gtap_amd.GtapError):  # ends early: queue overflow
+                gtap_amd.spmv(rp, ci, va, np.ones(50000), 1000)
+    finally:
+        st.close()
+
+
+def test_statistics_rows_are_whole():
+    """A launch writes every worker's whole statistics row: nothing of an earlier launch shows."""
+    print("case statistics rows of thread, block and thread launches in turn", flush=True)
+    _, s0 = gtap_amd.nqueens_cutoff(9, 4)
+    _, s1 = gtap_amd.cilksort(oracle.gen_keys_u32(40_000, 3))
+    ws = gtap_amd.worker_stats()
+    assert ws.shape[0] == s1["workers"] and int(ws[:, 0].sum()) == s1["tasks_executed"]
+    assert np.all(ws[:, [8, 9, 10, 13, 14, 15]] == 0)
+    v, s2 = gtap_amd.fib(15)
+    assert v == oracle.fib(15) and s2["tasks_executed"] == 3 * oracle.fib(16) - 2
