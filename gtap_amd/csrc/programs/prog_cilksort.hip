@@ -20,9 +20,9 @@
 //                           merge-path searches run by the workgroup's threads in parallel, each
 //                           chunk a cilkmerge task; taskwait (the output is the same sorted run)
 //
-// Differences from the reference's thread-mode program: uint32 keys; the leaf is `n <= 4096`
-// keys sorted by a 256-thread workgroup (bitonic network in LDS) instead of `n < 64` keys by
-// one thread; merges below MERGE_LEAF keys are done by a workgroup with merge-path tiles
+// Differences from the reference's thread-mode program: uint32 keys; the leaf is `n <= 8192`
+// keys (or the caller's smaller limit) sorted by a 256-thread workgroup (bitonic network in LDS)
+// instead of `n < 64` keys by one thread; merges below MERGE_LEAF keys are done by a workgroup with merge-path tiles
 // (4096 outputs per tile, staged through LDS) instead of one thread. The output is the
 // unique sorted permutation of the input whatever the schedule.
 //
@@ -52,28 +52,60 @@ struct MergeArg {
     int64_t nb;
 };
 struct CilkArgs {
-    int64_t leaf;        // <= 4096
+    int64_t leaf;        // ranges of at most this many keys (<= kMaxLeaf) are sorted by one workgroup
     int64_t merge_leaf;  // merges of at most this many keys are done by one workgroup
 };
+constexpr int kMaxLeaf = 2 * kTile;
+// Slot of key e in a leaf sort's LDS array, for `per` keys a thread: 4 words of padding after each
+// thread's keys, so that threads reading their own keys 16 bytes at a time meet all banks. The
+// keys e = q * kT + t of one thread lie leaf_stride apart.
+template <int per>
+__device__ __forceinline__ uint32_t leaf_slot(uint32_t e) { return e + e / (uint32_t)per * 4u; }
+template <int per>
+constexpr uint32_t leaf_stride = kT + kT / (uint32_t)per * 4u;
+constexpr int kLeafWords = kMaxLeaf + (int)kT * 4;
 
-struct Program {
-    static constexpr int kWavesPerSimd = 4;  // four 256-thread workgroups per CU
+struct CilkShared {
+    union {
+        struct {
+            uint32_t keys[kTile];
+            uint32_t out[kTile];
+        };
+        uint32_t sort[kLeafWords];  // leaf sort
+    };
+    int64_t split[kMaxFan + 2];
+};
+
+// Built for 4 waves per SIMD (four 256-thread workgroups per CU, 128 VGPRs, 44 of them spilled) and
+// for 3 (no spills to speak of): while the sort does not fill the chip a task's own time counts,
+// 20011 keys 116 / 108 us, 5M keys 719 / 706 us; beyond it more workgroups do, 20M keys 1398 / 1466 us,
+// 64M keys 3228 / 3474 us.
+template <int kWaves>
+struct ProgramT {
+    static constexpr int kWavesPerSimd = kWaves;
     static constexpr int kFrameWords = 10;
     static constexpr uint32_t kMaxFunc = F_MERGE;
     static constexpr uint32_t kFrameBytes = 40;
     using Args = CilkArgs;
-    struct Shared {
-        uint32_t keys[kTile];
-        uint32_t out[kTile];
-        int64_t split[kMaxFan + 2];
-    };
+    using Shared = CilkShared;
     template <class B>
     __device__ __forceinline__ static void run(B& blk);
 };
+using Program = ProgramT<4>;
+using SmallProgram = ProgramT<3>;
+constexpr int64_t kSmallKeys = 8 << 20;
 
 // keys live in device memory (the caller's arrays and the scratch buffer)
 __device__ __forceinline__ uint32_t ldk(const uint32_t* p) { return gld32(p); }
 __device__ __forceinline__ void stk(uint32_t* p, uint32_t v) { gst32(p, v); }
+
+// A task's arguments and the tile splits are the same for every thread, but come from LDS: as
+// scalars they cost no vector registers, and key addresses are one scalar base and a 32-bit offset.
+template <typename T>
+__device__ __forceinline__ T scalar(T v) {
+    static_assert(sizeof(T) == 8, "pointers and 64-bit integers");
+    return __builtin_bit_cast(T, uniform(__builtin_bit_cast(uint64_t, v)));
+}
 
 // gtap_cilksort.cu:40-50: largest index with x[index] <= val, or -1.
 __device__ __forceinline__ int64_t binary_search_gm(const uint32_t* x, int64_t len, uint32_t val) {
@@ -101,86 +133,87 @@ __device__ __forceinline__ void cmpx(uint32_t& x, uint32_t& y, bool up) {
 // wave: every register of the thread meets the same register of that lane.
 __device__ __forceinline__ uint32_t xlane(uint32_t v, int m) { return (uint32_t)__shfl_xor((int)v, m, kWave); }
 
-// Workgroup sort of arr[0..n), n <= 4096: bitonic sort of 4096 slots (padded with 0xFFFFFFFF,
-// which sorts to the end and is never written back). Thread t owns slots 16t .. 16t+15 in
-// registers. A step with partner distance j pairs slot s with s ^ j:
-//   j < 16          the partner is in the same thread: registers;
-//   16 <= j < 1024  the partner is register (s & 15) of lane (lane ^ j/16) of the same wave:
-//                   a cross-lane exchange, no barrier;
-//   j >= 1024       the partner is in another wave: through LDS with barriers (3 steps).
+// Workgroup sort of arr[0..n), n <= 256 per: bitonic sort of 256 per slots (padded with
+// 0xFFFFFFFF, which sorts to the end and is never written back). Thread t owns slots per t ..
+// per t + per - 1 in registers. A step with partner distance j pairs slot s with s ^ j:
+//   j < per            the partner is in the same thread: registers;
+//   per <= j < 64 per  the partner is the same register of lane (lane ^ j / per) of the same wave:
+//                      a cross-lane exchange, no barrier;
+//   j >= 64 per        the partner is in another wave: through LDS with barriers (3 steps).
 // Barriers here order LDS only (lds_barrier): the global loads and stores of a task need no
 // ordering among its threads, and the scheduler's barrier after the task waits for them.
-template <class B>
+template <int per, class B>
 __device__ void leaf_sort(B& blk, uint32_t* arr, int64_t n) {
-    uint32_t* k = blk.sh->keys;
+    lds_array<uint32_t> k = lds(blk.sh->sort);
     const uint32_t t = threadIdx.x;
+    const uint32_t at = leaf_slot<per>(t), cnt = (uint32_t)n;
     {
-        uint32_t r[kPer];
+        uint32_t r[per];
 #pragma unroll
-        for (int q = 0; q < kPer; ++q) {
+        for (int q = 0; q < per; ++q) {
             const uint32_t e = (uint32_t)q * kT + t;
-            r[q] = (int64_t)e < n ? ldk(arr + e) : 0xFFFFFFFFu;
+            r[q] = e < cnt ? ldk(arr + e) : 0xFFFFFFFFu;
         }
 #pragma unroll
-        for (int q = 0; q < kPer; ++q) k[(uint32_t)q * kT + t] = r[q];
+        for (int q = 0; q < per; ++q) k[at + (uint32_t)q * leaf_stride<per>] = r[q];
     }
     lds_barrier();
-    uint32_t x[16];
-    const uint32_t g0 = 16u * t;  // global slot of x[0]
+    uint32_t x[per];
+    const uint32_t g0 = (uint32_t)per * t;           // global slot of x[0]
+    const uint32_t own = leaf_slot<per>(g0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = k[g0 + (uint32_t)i];
-    // sizes 2..16: entirely inside each thread's 16 slots
+    for (int i = 0; i < per; ++i) x[i] = k[own + (uint32_t)i];
+    // sizes 2..per: entirely inside each thread's slots
 #pragma unroll
-    for (uint32_t size = 2; size <= 16; size <<= 1) {
+    for (uint32_t size = 2; size <= (uint32_t)per; size <<= 1) {
 #pragma unroll
         for (uint32_t j = size >> 1; j > 0; j >>= 1) {
 #pragma unroll
-            for (uint32_t i = 0; i < 16; ++i) {
+            for (uint32_t i = 0; i < (uint32_t)per; ++i) {
                 if ((i & j) == 0) cmpx(x[i], x[i + j], ((g0 + i) & size) == 0);
             }
         }
     }
-    for (uint32_t size = 32; size <= (uint32_t)kTile; size <<= 1) {
+    for (uint32_t size = 2u * per; size <= (uint32_t)per * kT; size <<= 1) {
         const bool up = (g0 & size) == 0;  // direction of this thread's slots at this size
-        for (uint32_t j = size >> 1; j >= 16; j >>= 1) {
-            const uint32_t m = j / 16;  // partner thread = t ^ m
+        for (uint32_t m = size / (2u * per); m >= 1; m >>= 1) {  // partner thread = t ^ m
             const bool low = (t & m) == 0;
             const bool keep_min = (low == up);
-            if (j >= 1024) {
+            if (m >= (uint32_t)kWave) {
                 lds_barrier();  // every thread has read the previous contents
 #pragma unroll
-                for (int i = 0; i < 16; ++i) k[g0 + (uint32_t)i] = x[i];
+                for (int i = 0; i < per; ++i) k[own + (uint32_t)i] = x[i];
                 lds_barrier();
-                const uint32_t p0 = 16u * (t ^ m);
+                const uint32_t p0 = leaf_slot<per>((uint32_t)per * (t ^ m));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < per; ++i) {
                     const uint32_t y = k[p0 + (uint32_t)i];
                     x[i] = keep_min ? (x[i] < y ? x[i] : y) : (x[i] < y ? y : x[i]);
                 }
             } else {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < per; ++i) {
                     const uint32_t y = xlane(x[i], (int)m);
                     x[i] = keep_min ? (x[i] < y ? x[i] : y) : (x[i] < y ? y : x[i]);
                 }
             }
         }
 #pragma unroll
-        for (uint32_t j = 8; j > 0; j >>= 1) {
+        for (uint32_t j = (uint32_t)per / 2; j > 0; j >>= 1) {
 #pragma unroll
-            for (uint32_t i = 0; i < 16; ++i) {
+            for (uint32_t i = 0; i < (uint32_t)per; ++i) {
                 if ((i & j) == 0) cmpx(x[i], x[i + j], up);
             }
         }
     }
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) k[g0 + (uint32_t)i] = x[i];
+    for (int i = 0; i < per; ++i) k[own + (uint32_t)i] = x[i];
     lds_barrier();
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
+    for (int q = 0; q < per; ++q) {
         const uint32_t e = (uint32_t)q * kT + t;
-        if ((int64_t)e < n) stk(arr + e, k[e]);
+        if (e < cnt) stk(arr + e, k[at + (uint32_t)q * leaf_stride<per>]);
     }
 }
 
@@ -259,10 +292,13 @@ __device__ void block_split_search(LDA lda, int64_t na, LDB ldb, int64_t nb, int
 __device__ __forceinline__ void load_tile(const uint32_t* a, int64_t i0, int64_t la, const uint32_t* b, int64_t j0,
                                           int64_t lb, uint32_t (&r)[kPer]) {
     const uint32_t t = threadIdx.x;
+    const uint32_t* pa = a + i0;
+    const uint32_t* pb = b + j0;
+    const uint32_t na = (uint32_t)la, n = (uint32_t)(la + lb);  // <= kTile
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-        const int64_t e = (int64_t)q * kT + t;
-        r[q] = e < la ? ldk(a + i0 + e) : (e < la + lb ? ldk(b + j0 + (e - la)) : 0u);
+        const uint32_t e = (uint32_t)q * kT + t;
+        r[q] = e < na ? ldk(pa + e) : (e < n ? ldk(pb + (e - na)) : 0u);
     }
 }
 
@@ -285,7 +321,7 @@ __device__ __forceinline__ int32_t merge_path_lds(const uint32_t* A, int32_t la,
 // a register, so each output costs one LDS load.
 template <class B>
 __device__ void leaf_merge(B& blk, const uint32_t* a, int64_t na, const uint32_t* b, int64_t nb, uint32_t* dst) {
-    typename Program::Shared* sh = blk.sh;
+    CilkShared* sh = blk.sh;
     const uint32_t t = threadIdx.x;
     const int64_t total = na + nb;
     auto ga = [a](int64_t i) { return ldk(a + i); };
@@ -297,7 +333,7 @@ __device__ void leaf_merge(B& blk, const uint32_t* a, int64_t na, const uint32_t
         const int ntl = ntiles_here < 16 ? (int)ntiles_here : 16;
         if (t == 0) sh->split[0] = carry;
         block_split_search(ga, na, gb, nb, base + kTile, kTile, ntl, sh->split + 1);
-        carry = sh->split[ntl];
+        carry = scalar(sh->split[ntl]);
         // The splits of sorted inputs are monotone along both inputs; anything else (unsorted
         // runs) would index outside the tile, so it is reported and the merge abandoned.
         bool ok = true;
@@ -314,21 +350,21 @@ __device__ void leaf_merge(B& blk, const uint32_t* a, int64_t na, const uint32_t
         }
         uint32_t r[kPer];
         {
-            const int64_t i0 = sh->split[0], i1 = sh->split[1];
+            const int64_t i0 = scalar(sh->split[0]), i1 = scalar(sh->split[1]);
             const int64_t d0 = base, d1 = (d0 + kTile < total) ? d0 + kTile : total;
             load_tile(a, i0, i1 - i0, b, d0 - i0, (d1 - i1) - (d0 - i0), r);
         }
         for (int ti = 0; ti < ntl; ++ti) {
             const int64_t d0 = base + (int64_t)ti * kTile;
             const int64_t d1 = (d0 + kTile < total) ? d0 + kTile : total;
-            const int64_t i0 = sh->split[ti], i1 = sh->split[ti + 1];
+            const int64_t i0 = scalar(sh->split[ti]), i1 = scalar(sh->split[ti + 1]);
             const int32_t la = (int32_t)(i1 - i0), lb = (int32_t)((d1 - i1) - (d0 - i0));
 #pragma unroll
             for (int q = 0; q < kPer; ++q) sh->keys[(uint32_t)q * kT + t] = r[q];
             lds_barrier();
             if (ti + 1 < ntl) {  // next tile's inputs in flight during this merge
                 const int64_t e0 = d1, e1 = (e0 + kTile < total) ? e0 + kTile : total;
-                const int64_t n0 = sh->split[ti + 1], n1 = sh->split[ti + 2];
+                const int64_t n0 = scalar(sh->split[ti + 1]), n1 = scalar(sh->split[ti + 2]);
                 load_tile(a, n0, n1 - n0, b, e0 - n0, (e1 - n1) - (e0 - n0), r);
             }
             const uint32_t* K = sh->keys;  // A = K[0..la), B = K[la..la+lb)
@@ -378,15 +414,17 @@ __device__ void leaf_merge(B& blk, const uint32_t* a, int64_t na, const uint32_t
 template <class B>
 __device__ void sort_task(B& blk) {
     const CilkArgs& g = *blk.args;
-    uint32_t* arr = blk.template arg<uint32_t*>(0);
-    uint32_t* tmp = blk.template arg<uint32_t*>(8);
-    const int64_t n = blk.template arg<int64_t>(16);
+    uint32_t* arr = scalar(blk.template arg<uint32_t*>(0));
+    uint32_t* tmp = scalar(blk.template arg<uint32_t*>(8));
+    const int64_t n = scalar(blk.template arg<int64_t>(16));
     const int64_t len12 = n / 2, len1 = len12 / 2, len2 = len12 - len1;
     const int64_t len34 = n - len12, len3 = len34 / 2, len4 = len34 - len3;
     switch (blk.get_state()) {
         case 0:
             if (n <= g.leaf) {
-                leaf_sort(blk, arr, n);
+                if (n <= 8 * (int64_t)kT) leaf_sort<8>(blk, arr, n);
+                else if (n <= 16 * (int64_t)kT) leaf_sort<16>(blk, arr, n);
+                else leaf_sort<32>(blk, arr, n);
                 blk.finish();
                 return;
             }
@@ -422,11 +460,11 @@ __device__ void sort_task(B& blk) {
 template <class B>
 __device__ void merge_task(B& blk) {
     const CilkArgs& g = *blk.args;
-    const uint32_t* a = blk.template arg<const uint32_t*>(0);
-    const uint32_t* b = blk.template arg<const uint32_t*>(8);
-    uint32_t* dst = blk.template arg<uint32_t*>(16);
-    int64_t na = blk.template arg<int64_t>(24);
-    int64_t nb = blk.template arg<int64_t>(32);
+    const uint32_t* a = scalar(blk.template arg<const uint32_t*>(0));
+    const uint32_t* b = scalar(blk.template arg<const uint32_t*>(8));
+    uint32_t* dst = scalar(blk.template arg<uint32_t*>(16));
+    int64_t na = scalar(blk.template arg<int64_t>(24));
+    int64_t nb = scalar(blk.template arg<int64_t>(32));
     if (blk.get_state() != 0) {
         blk.finish();
         return;
@@ -453,7 +491,7 @@ __device__ void merge_task(B& blk) {
     // searches run in parallel (one per chunk boundary), and the chunks are spawned as merge
     // tasks: one search latency per level instead of one per halving.
     {
-        typename Program::Shared* sh = blk.sh;
+        CilkShared* sh = blk.sh;
         const int64_t total = na + nb;
         int64_t fan = (total + g.merge_leaf - 1) / g.merge_leaf;
         if (fan > kMaxFan) fan = kMaxFan;
@@ -484,8 +522,9 @@ __device__ void merge_task(B& blk) {
     blk.finish();
 }
 
+template <int kWaves>
 template <class B>
-__device__ __forceinline__ void Program::run(B& blk) {
+__device__ __forceinline__ void ProgramT<kWaves>::run(B& blk) {
     if (blk.func == F_SORT) sort_task(blk);
     else merge_task(blk);
 }
@@ -498,8 +537,9 @@ static_assert(CilkProgram::kFrameBytes + gtap::kHdrBytes <= gtap::host::kBuiltin
 static_assert(CilkProgram::kFrameWords <= 16, "block frame cache holds 16 words");
 
 // Sorts n uint32 keys in place (device buffers keys and tmp, n elements each).
-// leaf <= 4096 keys are sorted by one workgroup in LDS (0 -> 4096); merges of at most
-// merge_leaf keys are done by one workgroup (0 -> 32768).
+// leaf <= 4096 keys are sorted by one workgroup in LDS (0 -> 4096; at 4096, ranges of up to 8192
+// are); merges of at most merge_leaf keys are done by one workgroup (0 -> 32768; at most 4096 to
+// 16384 for sorts of up to 32M keys).
 // Replaces the program of evaluation/2-comparison/cilksort/gtap_cilksort.cu:169-281.
 extern "C" int gtap_cilksort(uint32_t* keys, uint32_t* tmp, int64_t n, int64_t leaf, int64_t merge_leaf,
                              gtap_run_stats* stats) {
@@ -508,6 +548,12 @@ extern "C" int gtap_cilksort(uint32_t* keys, uint32_t* tmp, int64_t n, int64_t l
     if (leaf <= 0) leaf = 4096;
     if (merge_leaf <= 0) merge_leaf = 32768;
     if (leaf > cilk::kTile) return host::invalid_argument("gtap_cilksort: leaf must be <= 4096");
+    // A few workgroups merging long runs leave the others idle: with n keys no merge above `most`
+    // stays whole. Measured (us, 4096 / 8192 / 16384 / 32768): 1M keys 418 / 426 / 458 / 550, 4M 635 /
+    // 631 / 671 / 803, 16M 1298 / 1170 / 1169 / 1288, 64M 4424 / 3821 / 3487 / 3340; 20011 keys 139 /
+    // 145 / 147 / 149.
+    const int64_t most = n <= (2 << 20) ? 4096 : (n <= (8 << 20) ? 8192 : (n <= (32 << 20) ? 16384 : merge_leaf));
+    if (merge_leaf > most) merge_leaf = most;
     if (merge_leaf < 3) merge_leaf = 3;
     if (n == 0) {
         if (stats) memset(stats, 0, sizeof(*stats));
@@ -515,7 +561,11 @@ extern "C" int gtap_cilksort(uint32_t* keys, uint32_t* tmp, int64_t n, int64_t l
     }
     cilk::SortArg root{keys, tmp, n};
     gtap_job job = host::make_job(cilk::F_SORT, 0, &root, sizeof(root));
-    return host::run_single_block_job<CilkProgram>(cilk::CilkArgs{leaf, merge_leaf}, job, nullptr, stats);
+    // With the largest leaf, a range of up to two tiles is sorted whole, not cut into four short runs.
+    const int64_t top = leaf == cilk::kTile ? (int64_t)cilk::kMaxLeaf : leaf;
+    const cilk::CilkArgs args{top, merge_leaf};
+    if (n <= cilk::kSmallKeys) return host::run_single_block_job<cilk::SmallProgram>(args, job, nullptr, stats);
+    return host::run_single_block_job<CilkProgram>(args, job, nullptr, stats);
 }
 
 namespace gtap {

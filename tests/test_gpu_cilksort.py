@@ -44,3 +44,28 @@ def test_cilksort_benchmark_keys():
     keys = gtap_amd.gen_keys(n)  # gen_vector keys, seed 123456789
     out, st = gtap_amd.cilksort(keys)
     assert np.array_equal(out, np.sort(keys))
+
+
+@pytest.mark.parametrize("n", [7, 256, 2047, 2048, 2049, 4096, 4097, 8191, 8192, 8193, 16384, 32768, 32769, 40_000])
+@pytest.mark.parametrize("leaf", [4096, 2048, 3000])
+def test_cilksort_leaf_sizes(n, leaf):
+    """Leaf sorts of 8, 16 and 32 keys a thread at their limits, keys equal to the padding value,
+    runs in both directions and ties."""
+    print(f"case cilksort leaf sizes n={n} leaf={leaf}", flush=True)
+    rng = np.random.default_rng(n + leaf)
+    for keys in (rng.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32),
+                 np.full(n, 0xFFFFFFFF, dtype=np.uint32),
+                 np.where(rng.random(n) < 0.5, 0xFFFFFFFF, 0).astype(np.uint32),
+                 np.arange(n, dtype=np.uint32)[::-1].copy(),
+                 rng.integers(0, 3, n).astype(np.uint32)):
+        out, _ = gtap_amd.cilksort(keys, leaf=leaf)
+        assert np.array_equal(out, np.sort(keys))
+
+
+@pytest.mark.parametrize("n", [(2 << 20) + 1, (8 << 20), (8 << 20) + 1, (32 << 20) + 5])
+def test_cilksort_size_rules(n):
+    """One size on each side of the rules that choose the largest merge and the kernel build."""
+    print(f"case cilksort size rules n={n}", flush=True)
+    keys = np.random.default_rng(n).integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)
+    out, _ = gtap_amd.cilksort(keys)
+    assert np.array_equal(out, np.sort(keys))
