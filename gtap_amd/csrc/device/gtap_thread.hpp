@@ -1140,12 +1140,13 @@ __device__ __forceinline__ bool window_append(const GtapDev& dev, WaveCtxOf<P>* 
 
 // ------------------------------------------------------------------ spawns of a whole round
 // Spawns the children of a round's tasks together, from run_coop: lane l's task (func, tid) gets
-// `count` children of an additive join on lane queue QQ, the i-th with arguments next(i). All
+// `count` children on lane queue QQ, of an additive join or detached, the i-th with arguments
+// next(i). All
 // lanes take part, so the id stack's top, the queue's tail and its window masks are wave-uniform
 // and stay in scalar registers from one child index to the next. Spawning inside run(), where
 // only some lanes are active, reads and writes them in LDS for every child, a chain of about 600
 // cycles each: a round of n-queens(14) spent 2.1 us in task bodies that way, and 1.3 us this way.
-template <class P, int QQ, typename A, class Next>
+template <class P, int QQ, bool kJoin, typename A, class Next>
 __device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next next) {
     static_assert(sizeof(A) % 8 == 0 && sizeof(A) / 4 <= P::kFrameWords, "arguments must fit the loaded frame");
     static_assert(QQ < CtxShape<P>::kQL, "a lane queue");
@@ -1179,8 +1180,8 @@ __device__ __forceinline__ void spawn_round(Lane<P>& L, uint32_t count, Next nex
             const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
             uint32_t* d = &w->desc[QQ][(t0 + r) & (kWave - 1)][0];
             vst(&d[0], hdr_word0(L.func, 0, QQ));
-            vst(&d[1], L.tid);
-            vst(&d[2], kResSum);
+            vst(&d[1], kJoin ? L.tid : kNoParent);
+            vst(&d[2], kJoin ? kResSum : 0u);
 #pragma unroll
             for (int k = 0; k < (int)(sizeof(A) / 4); ++k) vst(&d[3 + k], src[k]);
         }

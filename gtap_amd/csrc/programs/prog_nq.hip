@@ -146,7 +146,7 @@ __device__ __forceinline__ void ProgramT<kSum>::run_coop(L& lane, uint64_t mask,
     uint32_t avail = lane.coop ? lane.coop_arg : 0u;
     const int32_t row = (int32_t)lane.frame[0];
     const uint32_t cols = lane.frame[1], diag = lane.frame[2], anti = lane.frame[3];
-    spawn_round<ProgramT<kSum>, 0, NqArg>(lane, (uint32_t)popc32(avail), [&](uint32_t) {
+    spawn_round<ProgramT<kSum>, 0, true, NqArg>(lane, (uint32_t)popc32(avail), [&](uint32_t) {
         const uint32_t p = avail & (0u - avail);
         avail -= p;
         return NqArg{row + 1, cols | p, (diag | p) << 1, (anti | p) >> 1};
@@ -172,56 +172,70 @@ struct CutoffArgs {
     int32_t cutoff;
 };
 
-// Solutions below (row, cols, left, right), row < n: a depth-first walk that lives in registers.
-// The two diagonal sets are kept in board coordinates (bit col - row + n - 1 and bit
-// col + row, at most bit 30 for n <= 16), so a step back is the same exclusive or as the step
-// forward, and the columns of the path are 4 bits each in one 64-bit word: no stack in memory
-// (with one, as four private arrays, every step waited for scratch memory and the walks of a
-// round took 113 us at n = 15). After a step back the columns not yet tried are those above the
-// one taken back. Placements in row n - 2 are not stepped into: the last row's free columns
-// are counted from there.
-__device__ __forceinline__ int32_t nq_serial(int32_t row, int32_t n, uint32_t cols, uint32_t left, uint32_t right) {
-    const uint32_t mask = (1u << n) - 1u;
-    uint32_t avail = mask & ~(cols | left | right);
-    if (row == n - 1) return popc32(avail);
-    const int32_t top = n - 1;
-    uint32_t dl = (left & mask) << (top - row), dr = (right & mask) << row;
-    uint64_t path = 0;
-    int32_t r = row, count = 0;
-    while (true) {
+// A lane's share of the sequential search: a depth-first walk that lives in registers. The two
+// diagonal sets are kept in board coordinates (bit col - row + n - 1 and bit col + row, at most
+// bit 30 for n <= 16), so a step back is the same exclusive or as the step forward, and the
+// columns of the path are 4 bits each in one 64-bit word: no stack in memory (with one, as four
+// private arrays, every step waited for scratch memory and the walks of a round took 113 us at
+// n = 15). The walk starts at `base` with the columns `rem` of that row to try, and may lose some of
+// those it has not come to (another lane takes them). Placements in row n - 2 are not stepped
+// into: the last row's free columns are counted from there.
+struct Walk {
+    uint32_t cols, dl, dr, avail, rem;
+    uint64_t path;
+    int32_t r, base;
+
+    __device__ __forceinline__ bool active() const { return avail != 0u || r != base; }
+    __device__ __forceinline__ void start(int32_t row, uint32_t c, uint32_t l, uint32_t d, uint32_t todo) {
+        base = r = row;
+        cols = c;
+        dl = l;
+        dr = d;
+        rem = avail = todo;
+        path = 0;
+    }
+    // One placement or one step back; returns the solutions it counted.
+    __device__ __forceinline__ int32_t step(int32_t top, uint32_t mask) {
         const bool fwd = avail != 0u;
-        if (!fwd && r == row) break;
         const int32_t at = fwd ? r : r - 1;  // the row whose queen is placed or taken back
         const uint32_t c = fwd ? (uint32_t)__builtin_ctz(avail | 0x80000000u) : (uint32_t)path & 15u;
         const uint32_t p = 1u << c;
         const uint32_t cols1 = cols ^ p, dl1 = dl ^ (p << (top - at)), dr1 = dr ^ (p << at);
         const int32_t r1 = fwd ? r + 1 : at;
         const uint32_t free1 = mask & ~(cols1 | (dl1 >> (top - r1)) | (dr1 >> r1));
+        rem = fwd && at == base ? rem ^ p : rem;
         if (fwd && r1 == top) {
-            count += popc32(free1);
             avail ^= p;
-        } else {
-            cols = cols1;
-            dl = dl1;
-            dr = dr1;
-            r = r1;
-            path = fwd ? (path << 4) | c : path >> 4;
-            avail = fwd ? free1 : free1 & (~1u << c);
+            return popc32(free1);
         }
+        cols = cols1;
+        dl = dl1;
+        dr = dr1;
+        r = r1;
+        path = fwd ? (path << 4) | c : path >> 4;
+        avail = fwd ? free1 : (r1 == base ? rem : free1 & (~1u << c));
+        return 0;
     }
-    return count;
-}
+};
+constexpr int kWalkSteps = 4;   // steps between two looks at the idle lanes
+// Idle lanes that make the busy ones share: N = 14, 8 / 16 / 24: 429 / 415 / 411 us; N = 15: 1154 / 1147 /
+// 1162 us (without sharing 465 and 1438 us).
+constexpr int kWalkIdle = 16;
 
 struct CutoffProgram {
     static constexpr int kQueues = 1;
     static constexpr bool kNoTaskwait = true;
     static constexpr uint32_t kIdleProbes = 2;
     static constexpr bool kLaneSum = true;
+    static constexpr bool kCoop = true;  // children and searches: run_coop
     static constexpr int kWavesPerSimd = 4;
     static constexpr int kFrameWords = 4;  // row, cols, left, right
     static constexpr uint32_t kMaxFunc = F_NQ;
     static constexpr uint32_t kFrameBytes = 16;
     using Args = CutoffArgs;
+    struct WaveShared {
+        int32_t lane[kWave];  // the lanes that give a column away
+    };
     template <class L>
     __device__ __forceinline__ static void run(L& lane) {
         const CutoffArgs& g = *lane.args;
@@ -229,22 +243,83 @@ struct CutoffProgram {
         const uint32_t cols = lane.template arg<uint32_t>(4);
         const uint32_t left = lane.template arg<uint32_t>(8);
         const uint32_t right = lane.template arg<uint32_t>(12);
-        int32_t found = 0;
+        const uint32_t avail = ((1u << g.n) - 1u) & ~(cols | left | right);
         if (row == g.n) {
-            found = 1;
-        } else if (row > g.cutoff) {
-            found = nq_serial(row, g.n, cols, left, right);
+            lane.total += 1u;
+        } else if (row == g.n - 1 && row > g.cutoff) {
+            lane.total += (uint32_t)popc32(avail);
         } else {
-            const uint32_t mask = (g.n < 32) ? ((1u << g.n) - 1u) : 0xFFFFFFFFu;
-            uint32_t avail = mask & ~(cols | left | right);
-            while (avail) {
+            lane.coop = avail != 0u;  // the children, or the search: run_coop
+            lane.coop_arg = avail;
+        }
+        __gtap_finish_task(lane);
+    }
+    // Rows up to the cutoff: a child task per free column. Below it: the round's searches, on all
+    // lanes. Their lengths differ (a mean of 50 steps and a longest of 134 in a round at n = 15,
+    // cutoff 7), so once kWalkIdle lanes have nothing to do, each takes one of the first row's
+    // columns that a busy lane has not come to.
+    template <class L>
+    __device__ __forceinline__ static void run_coop(L& lane, uint64_t mask, WaveShared* sh) {
+        (void)mask;
+        const CutoffArgs& g = *lane.args;
+        const int32_t l = lane_id();
+        const int32_t row = (int32_t)lane.frame[0];
+        const uint32_t cols = lane.frame[1], left = lane.frame[2], right = lane.frame[3];
+        const bool walks = lane.coop && row > g.cutoff;
+        uint32_t avail = lane.coop && !walks ? lane.coop_arg : 0u;
+        if (ballot(avail != 0u)) {
+            spawn_round<CutoffProgram, 0, false, NqArg>(lane, (uint32_t)popc32(avail), [&](uint32_t) {
                 const uint32_t p = avail & (0u - avail);
                 avail -= p;
-                __gtap_spawn_task_detached(lane, F_NQ, 0, NqArg{row + 1, cols | p, (left | p) << 1, (right | p) >> 1});
-            }
+                return NqArg{row + 1, cols | p, (left | p) << 1, (right | p) >> 1};
+            });
         }
-        lane.total += (uint32_t)found;
-        __gtap_finish_task(lane);
+        if (ballot(walks) == 0) return;
+        const int32_t top = g.n - 1;
+        const uint32_t board = (1u << g.n) - 1u;
+        Walk w;
+        w.start(0, 0u, 0u, 0u, 0u);
+        uint32_t bc = 0, bl = 0, bd = 0;  // the board that w starts from
+        if (walks) {
+            bc = cols;
+            bl = (left & board) << (top - row);
+            bd = (right & board) << row;
+            w.start(row, bc, bl, bd, lane.coop_arg);
+        }
+        uint32_t found = 0;
+        while (true) {
+#pragma unroll 1
+            for (int k = 0; k < kWalkSteps; ++k)
+                if (w.active()) found += (uint32_t)w.step(top, board);
+            const uint64_t idle = ballot(!w.active());
+            if (idle == ~0ull) break;
+            if (popc(idle) < kWalkIdle) continue;
+            const bool gives = w.active() && (w.r > w.base ? w.rem != 0u : (w.rem & (w.rem - 1u)) != 0u);
+            const uint64_t donors = ballot(gives);
+            if (donors == 0) continue;
+            const int32_t pairs = popc(idle) < popc(donors) ? popc(idle) : popc(donors);
+            const int32_t rank = w.active() ? rank_in(donors) : rank_in(idle);
+            uint32_t part = 0;  // the column given away: the last one
+            if (gives && rank < pairs) {
+                part = 1u << (31 - __builtin_clz(w.rem));
+                w.rem ^= part;
+                if (w.r == w.base) w.avail = w.rem;
+                lds(sh->lane)[rank] = l;
+            }
+            wave_sync();
+            const bool takes = !w.active() && rank < pairs;
+            const int32_t src = takes ? lds(sh->lane)[rank] : l;
+            const uint32_t c1 = shfl(bc, src), l1 = shfl(bl, src), d1 = shfl(bd, src);
+            const uint32_t what = shfl(part | ((uint32_t)w.base << 16), src);
+            if (takes) {
+                bc = c1;
+                bl = l1;
+                bd = d1;
+                w.start((int32_t)(what >> 16), bc, bl, bd, what & 0xFFFFu);
+            }
+            wave_sync();
+        }
+        lane.total += found;
     }
 };
 
