@@ -149,8 +149,9 @@ __device__ __forceinline__ void spawn_hits(T& t, const BfsArgs& g, ExpandShared*
 // `begin` (none: 0), whose vertices get depth nd. The ranges form one flat sequence of edges and
 // lane l takes edges b + 64 j + l of it, so every lane has work until the last edges, a round
 // lasts as long as its edges and not as its longest range, and loads are contiguous. (With one
-// range per lane, 16 edges at a time, a round of R-MAT 22 took 22.6 us for 717 edges on average,
-// four chains of dependent loads for the longest range.)
+// range per lane, 16 edges at a time, a round of R-MAT 22 took 22.6 us for some 700 edges, up to
+// four chains of dependent loads for the longest range; now 17.3 us for 610. R-MAT 18 with one
+// queue: 367 us then, 249 us now.)
 //
 // kWindows column loads per lane are in flight together, then their probes, then their atomics.
 // A plain load of depth[u] filters the atomics: depths only decrease, so a stale cached value is

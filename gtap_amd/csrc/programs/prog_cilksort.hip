@@ -77,7 +77,7 @@ struct CilkShared {
 };
 
 // Built for 4 waves per SIMD (four 256-thread workgroups per CU, 128 VGPRs, 44 of them spilled) and
-// for 3 (no spills to speak of): while the sort does not fill the chip a task's own time counts,
+// for 3 (168 VGPRs, none spilled): while the sort does not fill the chip a task's own time counts,
 // 20011 keys 116 / 108 us, 5M keys 719 / 706 us; beyond it more workgroups do, 20M keys 1398 / 1466 us,
 // 64M keys 3228 / 3474 us.
 template <int kWaves>
