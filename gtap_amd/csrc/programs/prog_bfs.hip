@@ -96,10 +96,18 @@ struct Program {
     using Args = BfsArgs;
     using WaveShared = ExpandShared;
     static constexpr bool kCoop = true;  // the edges of a round are scanned by run_coop
-    // With one queue a wave holds few tasks while the search spreads, and 32 a batch spread it
-    // sooner: R-MAT 18, 64 / 32 / 16 a batch: 297 / 258 / 286 us, R-MAT 22: 1050 / 1048 / 1288 us. With
-    // four, each queue's batch is smaller anyway: R-MAT 22, 64 / 32: 1116 / 1196 us.
-    __device__ __forceinline__ static uint32_t batch_cap(const Args&) { return NQ == 1 ? 32u : 64u; }
+    // With one queue a wave holds few tasks while the search spreads, and batches of 32 tasks of up
+    // to 64 edges spread it sooner: R-MAT 18, 64 / 32 / 16 a batch: 297 / 258 / 286 us. Ranges cut
+    // smaller than that make a batch of 32 too little work for its round (R-MAT 22 in ranges of 32
+    // edges, 32 / 64 a batch: 1212 / 995 us; of 16 edges: 1700 / 1236 us), so a batch holds 2048
+    // edges' worth of tasks. (One range per lane without the flat scan took 1050 and 1152 us there:
+    // ranges of 16 edges are the one size that it scans faster.) With four queues, each queue's
+    // batch is smaller anyway: R-MAT 22, 64 / 32: 1116 / 1196 us.
+    __device__ __forceinline__ static uint32_t batch_cap(const Args& g) {
+        if constexpr (NQ != 1) return (uint32_t)kWave;
+        const uint32_t n = g.split > 0 ? (uint32_t)(2048 / g.split) : (uint32_t)kWave;
+        return n < 32u ? 32u : (n > (uint32_t)kWave ? (uint32_t)kWave : n);
+    }
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
     template <class L>
