@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../device/gtap_block.hpp"
@@ -293,6 +294,25 @@ inline int replay_thread(const ThreadGraph& g, gtap_run_stats* stats) {
     if (int st = enqueue_summary(g.dev, R.stream, false)) return st;
     GTAP_HIP_TRY(hipStreamSynchronize(R.stream));
     return finish_launch(g.dev, g.blocks, stats);
+}
+
+// Fills a root's arguments and queue by the one-thread kernel `root` (a lowered module's, for
+// entry arguments that only have a value on the device). On the null stream, as a host-launched
+// entry is: behind the caller's writes of device variables. The result goes through the pinned summary.
+template <class... Params>
+int evaluate_root(void (*root)(gtap_job*, Params...), gtap_job& job, std::common_type_t<Params>... params) {
+    Runtime& R = rt();
+    if (!R.initialized) {
+        int st = gtap_initialize();
+        if (st) return st;
+    }
+    memset(&R.summary->job0, 0, sizeof(gtap_job));
+    hipLaunchKernelGGL(root, dim3(1), dim3(1), 0, nullptr, &R.summary_dev->job0, params...);
+    GTAP_HIP_TRY(hipGetLastError());
+    GTAP_HIP_TRY(hipStreamSynchronize(nullptr));
+    job.queue = R.summary->job0.queue;
+    memcpy(job.args, R.summary->job0.args, sizeof(job.args));
+    return 0;
 }
 
 // One job in slot 0 of the device job table; the root's return value goes to *result.

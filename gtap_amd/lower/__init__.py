@@ -916,6 +916,20 @@ __device__ __forceinline__ void {t.name}__load(L& lane, {t.name}__frame& fr) {{
             out.append(s)
         return "\n".join(out)
 
+    def _host_value(self, arg: "cl.Node", names) -> bool:
+        """Whether an entry argument has the same value in host code: arithmetic on literals and on
+        the kernel's own parameters (`names`), nothing loaded and nothing called."""
+        for n in arg.walk():
+            if n.kind == cl.DECL_REF_EXPR:
+                if n.spelling not in names:
+                    return False
+            elif n.kind == cl.UNARY_OPERATOR:
+                if self.text[n.start] not in "-+~!":
+                    return False
+            elif n.kind not in cl.HOST_VALUE_KINDS:
+                return False
+        return True
+
     def entry_kernels(self) -> Tuple[str, str]:
         """The host-launched `__global__` kernels with their entries, and the host helpers."""
         kern_txt, host_txt = [], []
@@ -977,7 +991,25 @@ extern "C" int gtap_launch_{k.spelling}(uint32_t grid, uint32_t block{sep}{cpara
     return (int)hipGetLastError();
 }}
 """)
-            largs = ", ".join(f"({v.type})({self.text[a.start:a.end]})" for v, a in zip(t.params, call.children[1:]))
+            names = {c.spelling for c in params}
+            if all(self._host_value(a, names) for a in call.children[1:]) and \
+                    set(re.findall(r"[A-Za-z_]\w*", p.queue or "")) <= names:
+                largs = ", ".join(f"({v.type})({self.text[a.start:a.end]})" for v, a in zip(t.params, call.children[1:]))
+                root = (f"const {t.name}__args gtap_root_args{{{largs}}};\n"
+                        f"    gtap_job job = ::gtap::host::make_job(F_{t.name}, (uint32_t)({p.queue or '0'}), &gtap_root_args, "
+                        f"sizeof(gtap_root_args));")
+            else:
+                # anything else (a device variable, a load) has its value on the device only
+                rsep = ", " if ptxt else ""
+                kern_txt.append(f"""// Root task of `{self.text[first.start:first.end]}`, for gtap_entry_{k.spelling}.
+__global__ void {k.spelling}__root(gtap_job* gtap_root{rsep}{ptxt}) {{
+    const {ns}::{t.name}__args gtap_root_args{{{args}}};
+    memcpy(gtap_root->args, &gtap_root_args, sizeof(gtap_root_args));
+    gtap_root->queue = (uint32_t)({p.queue or "0"});
+}}
+""")
+                root = (f"gtap_job job = ::gtap::host::make_job(F_{t.name}, 0u, nullptr, 0);\n"
+                        f"    if (const int rst = ::gtap::host::evaluate_root(&{k.spelling}__root, job{sep}{cnames})) return rst;")
             res = "" if t.ret_type == "void" else f"{t.ret_type}* result, "
             copy = "" if t.ret_type == "void" else f"    if (st == 0 && result) memcpy(result, &r, sizeof({t.ret_type}));\n"
             if self.mode == "block":
@@ -988,8 +1020,7 @@ extern "C" int gtap_launch_{k.spelling}(uint32_t grid, uint32_t block{sep}{cpara
 // by the library (the kernel's other statements are not run).
 extern "C" int gtap_entry_{k.spelling}({cparams}{sep}{res}gtap_run_stats* stats) {{
     using namespace {ns};
-    const {t.name}__args gtap_root_args{{{largs}}};
-    gtap_job job = ::gtap::host::make_job(F_{t.name}, (uint32_t)({p.queue or "0"}), &gtap_root_args, sizeof(gtap_root_args));
+    {root}
     int64_t r = 0;
     const int st = {run};
 {copy}    return st;

@@ -20,12 +20,16 @@ PARM_DECL = 10
 DECL_REF_EXPR = 101
 MEMBER_REF_EXPR = 102
 CALL_EXPR = 103
+UNARY_OPERATOR = 112
 ARRAY_SUBSCRIPT_EXPR = 113
 BINARY_OPERATOR = 114
 COMPOUND_STMT = 202
 FOR_STMT = 209
 RETURN_STMT = 214
 DECL_STMT = 231
+# unexposed (implicit casts), integer, floating and character literals, parentheses, binary operator,
+# ?:, C cast, bool literal
+HOST_VALUE_KINDS = (100, 106, 107, 110, 111, 114, 116, 117, 130)
 
 
 class _CXString(C.Structure):

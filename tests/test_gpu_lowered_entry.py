@@ -146,3 +146,28 @@ def test_launch_with_a_smaller_grid(mods):
     for grid in (1, 3, 17):
         assert m.launch("fib_kernel", [ctypes.c_int], 18, grid=grid) == 0
         assert m.get_symbol("d_fib_result", ctypes.c_longlong) == oracle.fib(18)
+
+
+@pytest.mark.parametrize("name,kernel", [("csort", "csort_kernel"), ("bsort", "bsort_kernel")])
+@pytest.mark.parametrize("n", [1, 33, 1000, 65_539])
+def test_library_launch_of_an_entry_with_device_variables(mods, name, kernel, n):
+    """gtap_entry_<kernel> reads the __device__ pointers of the entry call's arguments on the
+    device, with the values that the host set last."""
+    print(f"case gtap_entry_{kernel} n={n}", flush=True)
+    m = mods[name]
+    f = getattr(m.L, f"gtap_entry_{kernel}")
+    f.argtypes = [ctypes.c_int, ctypes.c_void_p]
+    f.restype = ctypes.c_int
+    for seed in (1, 2):
+        keys = oracle.gen_keys_u32(n, 40 * seed + n)
+        a = gtap_amd.DeviceBuffer.from_array(keys)
+        t = gtap_amd.DeviceBuffer(n * 4)
+        try:
+            m.set_symbol("g_keys", a.ptr, ctypes.c_uint64)
+            m.set_symbol("g_tmp", t.ptr, ctypes.c_uint64)
+            s = gtap_amd.RunStats()
+            assert f(n, ctypes.addressof(s)) == 0 and s.error_code == 0
+            assert np.array_equal(a.to_array(np.empty(n, dtype=np.uint32)), np.sort(keys))
+        finally:
+            a.free()
+            t.free()

@@ -176,6 +176,54 @@ def test_built_libraries_export_entries():
         del L, L2
 
 
+ENTRY_ARGS = """
+#include "gtap_thread.cuh"
+__device__ int* g_data;
+__constant__ int c_n;
+#define TWICE(x) (2 * (x))
+#pragma gtap function
+__device__ void visit(int* a, int n) {
+    if (n < 2) return;
+    #pragma gtap task
+    visit(a, n - 1);
+}
+__global__ void k(int* a, int n) {
+    #pragma gtap entry QUEUE
+    visit(ARGS);
+}
+"""
+
+
+def entry_function(text, kernel):
+    at = text.index(f'extern "C" int gtap_entry_{kernel}(')
+    return text[at:text.index("\n}\n", at)]
+
+
+@pytest.mark.parametrize("name,kernel,variables", [("csort", "csort_kernel", ("g_keys", "g_tmp")),
+                                                   ("bsort", "bsort_kernel", ("g_keys", "g_tmp"))])
+def test_entry_arguments_with_device_variables_are_read_on_the_device(name, kernel, variables):
+    """The name of a __device__ variable in host code is its host stand-in, not its value: a root
+    task built from it on the host would run on null pointers. Such arguments are evaluated by a
+    kernel, as the host-launched form does."""
+    text = lower.lower(read(f"{name}.gtap.cu"), f"{name}.gtap.cu", name)
+    host = entry_function(text, kernel)
+    assert not any(v in host.split("(kernel's")[0].split("{", 1)[1] for v in variables)
+    assert f"{kernel}__root" in host
+    at = text.index(f"__global__ void {kernel}__root(")
+    dev = text[at:text.index("\n}\n", at)]
+    assert all(v in dev for v in variables)
+
+
+@pytest.mark.parametrize("args,queue,on_device", [
+    ("a, n", "", False), ("a, -n + TWICE(3)", "", False), ("a, (int)(n / 2)", "queue(n % 2)", False),
+    ("g_data, n", "", True), ("a, c_n", "", True), ("a, *a", "", True), ("a, a[n]", "", True), ("&a[1], n", "", True),
+    ("g_data + 1, n + c_n", "", True), ("a, n", "queue(c_n)", True), ("a, load_L2(a)", "", True)])
+def test_entry_arguments_host_or_device(args, queue, on_device):
+    text = lower.lower(ENTRY_ARGS.replace("ARGS", args).replace("QUEUE", queue), "entry_args.cu", "entry_args")
+    assert ("__global__ void k__root(" in text) == on_device
+    assert ("k__root" in entry_function(text, "k")) == on_device
+
+
 PLAIN_MSORT = """
 #include "gtap_thread.cuh"
 __device__ int* g_data;
