@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "../device/gtap_abi.hpp"
+#include "../device/gtap_steps.hpp"
 #include "../host/gtap_launch.hpp"
 
 namespace gtap {
@@ -127,11 +128,11 @@ __device__ __forceinline__ void range_task(L& lane) {
 
 // The entries of the kPer * g of a row's entries that one step takes: this lane's columns and
 // values, entry j at offset first + j * g of a row of `length` entries from `begin`.
-__device__ __forceinline__ void load_entries(const SpmvArgs& a, int32_t begin, int32_t length, int32_t first, int32_t g,
+__device__ __forceinline__ void load_entries(const SpmvArgs& a, int32_t begin, uint32_t length, uint32_t first, uint32_t g,
                                              int32_t (&c)[kPer], double (&v)[kPer]) {
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
-        const int32_t e = first + j * g;
+        const uint32_t e = first + (uint32_t)j * g;
         c[j] = e < length ? __builtin_nontemporal_load(a.col_idx + begin + e) : -1;
         v[j] = e < length ? __builtin_nontemporal_load(a.val + begin + e) : 0.0;
     }
@@ -165,64 +166,69 @@ __device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveSh
     wave_sync();
     const int32_t rows = kWave / g, step = kPer * g, stride = step + 1;
     const int32_t slot = l / g, sub = l & (g - 1);
+    const uint32_t width = (uint32_t)g;
     lds_array<Entry> tile = lds(sh->tile);
     // The steps of all groups in one sequence, the next step's columns and values in flight
     // while the current one gathers and sums, over the end of a group too.
-    int32_t p0 = 0, b = 0;       // current step: the group's first row (of the m), its entries' offset
-    int32_t begin, length;       // this lane loads entries sub, sub + g, ... of row p0 + slot
-    int32_t row, left;           // and, among the first `rows` lanes, sums row p0 + l: entries left
+    int32_t p0 = 0;              // current step: the group's first row (of the m)
+    int32_t begin;               // this lane loads entries sub, sub + g, ... of a step of row p0 + slot
+    Steps load{0u, (uint32_t)step, 0u};
+    int32_t row;                 // and, among the first `rows` lanes, sums a step of row p0 + l
+    Steps add{0u, (uint32_t)step, 0u};
     bool sums;
     auto load_part = [&](int32_t p) {
         const bool on = p + slot < m;
         const int32_t src = lds(sh->src)[on ? p + slot : 0];
         begin = shfl((int32_t)lane.frame[kRowBegin], src);
-        length = shfl((int32_t)lane.frame[kRowLength], src);
-        if (!on) length = 0;
+        const uint32_t length = shfl(lane.frame[kRowLength], src);
+        load.n = on ? length : 0u;
     };
     auto sum_part = [&](int32_t p) {
         sums = l < rows && p + l < m;
         const int32_t own = lds(sh->src)[sums ? p + l : 0];
         row = shfl((int32_t)lane.frame[0], own);
-        left = shfl((int32_t)lane.frame[kRowLength], own);
-        if (!sums) left = 0;
+        const uint32_t length = shfl(lane.frame[kRowLength], own);
+        add.n = sums ? length : 0u;
+        add.at = 0u;
     };
     load_part(0);
     sum_part(0);
     double sum = 0.0;
     int32_t c[kPer];
     double v[kPer];
-    load_entries(a, begin, length, sub, g, c, v);
+    load_entries(a, begin, load.n, (uint32_t)sub, width, c, v);
     while (true) {
         double xv[kPer];
         bool bad = false;
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
-            const bool in = b + j * g + sub < length;
+            const bool in = load.at + (uint32_t)j * width + (uint32_t)sub < load.n;
             const bool valid = (uint32_t)c[j] < (uint32_t)a.cols;
             bad |= in && !valid;
             xv[j] = in && valid ? a.x[c[j]] : 0.0;
         }
         if (bad) GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, begin, a.cols);
-        const bool more = ballot(b + step < length) != 0;
-        b = more ? b + step : 0;
+        const bool more = ballot(load.more()) != 0;
+        load.at = more ? load.at + load.step : 0u;
         const int32_t p1 = more ? p0 : p0 + rows;
         if (!more && p1 < m) load_part(p1);
         int32_t c1[kPer];
         double v1[kPer];
-        if (p1 < m) load_entries(a, begin, length, b + sub, g, c1, v1);
+        if (p1 < m) load_entries(a, begin, load.n, load.at + (uint32_t)sub, width, c1, v1);
         wave_sync();  // the previous step's entries have been read
 #pragma unroll
         for (int j = 0; j < kPer; ++j) tile[slot * stride + j * g + sub] = Entry{v[j], xv[j]};
         wave_sync();
-        for (int32_t e = 0; e < step && e < left; e += kPer) {
+        const uint32_t left = add.left();
+        for (uint32_t e = 0; e < add.step && e < left; e += kPer) {
             Entry t[kPer];
 #pragma unroll
-            for (int j = 0; j < kPer; ++j) t[j] = tile[l * stride + e + j];
+            for (int j = 0; j < kPer; ++j) t[j] = tile[l * stride + (int32_t)e + j];
 #pragma unroll
             for (int j = 0; j < kPer; ++j)
-                if (e + j < left) sum = __builtin_fma(t[j].x, t[j].y, sum);
+                if (e + (uint32_t)j < left) sum = __builtin_fma(t[j].x, t[j].y, sum);
         }
-        left -= step;
+        add.next();
         if (!more) {
             if (sums) a.y[row] = sum;
             if (p1 >= m) break;

@@ -34,6 +34,7 @@
 #include <cstring>
 
 #include "../device/gtap_abi.hpp"
+#include "../device/gtap_steps.hpp"
 #include "../host/gtap_launch.hpp"
 
 namespace gtap {
@@ -135,6 +136,7 @@ __device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveSh
     const int32_t m = popc(mask);
     int32_t g = kWave;
     while (g * m > kWave) g >>= 1;
+    const uint32_t width = (uint32_t)g;
     if (lane.coop) vst(&sh->src[rank_in(mask)], l);
     wave_sync();
     const int32_t grp = l / g, sub = l % g;
@@ -147,25 +149,25 @@ __device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveSh
     const uint32_t seed = xs32((uint32_t)node ^ 0x9e3779b9u);
     double acc = 0.0;
     lds_array<double> buf = lds(&sh->v[grp * g * kCoopReads]);
-    const int32_t step = g * kCoopReads;
-    for (int32_t m0 = 0; ballot(m0 < mem_ops); m0 += step) {
+    for (Steps reads{(uint32_t)mem_ops, width * kCoopReads, 0u}; ballot(reads.on()); reads.next()) {
         double v[kCoopReads];
 #pragma unroll
         for (int j = 0; j < kCoopReads; ++j) {
-            const int32_t k = m0 + j * g + sub;
-            v[j] = k < mem_ops ? a.input[xs32(seed + (uint32_t)k * 747796405u) & a.input_mask] : 0.0;
+            const uint32_t k = reads.at + (uint32_t)j * width + (uint32_t)sub;
+            v[j] = k < reads.n ? a.input[xs32(seed + k * 747796405u) & a.input_mask] : 0.0;
         }
         wave_sync();  // the previous step's values have been read
 #pragma unroll
         for (int j = 0; j < kCoopReads; ++j) buf[j * g + sub] = v[j];
         wave_sync();
-        const int32_t cnt = mem_ops - m0 < step ? mem_ops - m0 : step;
+        const uint32_t cnt = reads.more() ? reads.step : reads.left();
 #pragma unroll 8
-        for (int32_t k = 0; k < cnt; ++k) acc += buf[k];
+        for (uint32_t k = 0; k < cnt; ++k) acc += buf[k];
     }
     uint32_t mix = 0;
+    const Steps its{(uint32_t)iters, width, (uint32_t)sub};
 #pragma unroll 4
-    for (int32_t it = sub; it < iters; it += g) mix ^= mix_term(seed, (uint32_t)it);
+    for (uint32_t k = 0, n = its.steps(); k < n; ++k) mix ^= mix_term(seed, its.at + k * width);
     for (int32_t d = g / 2; d > 0; d >>= 1) mix ^= (uint32_t)shfl((int32_t)mix, l ^ d);
     mix ^= (0x9e3779b9u ^ (uint32_t)node) + sat_u32(acc);
     if (on && sub == 0) a.out[node] = (double)mix;

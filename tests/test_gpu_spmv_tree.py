@@ -122,6 +122,16 @@ def test_tree_batch_sizes(height, mem_ops, iters):
     assert s["tasks_executed"] == 3 * (1 << height) - 2
 
 
+def test_tree_most_steps():
+    """One node with the most steps the argument holds: the lanes' walks (64 steps apart) end past
+    2^31 - 1."""
+    iters = 2**31 - 1
+    print(f"case tree height=0 iters={iters}", flush=True)
+    inp = G.tree_input(16, 3)
+    out, s = G.tree(0, 3, iters, inp)
+    assert s["error_code"] == 0 and np.array_equal(out, O.tree(0, 3, iters, inp))
+
+
 def test_bfs_on_graph_read_from_reference_format(tmp_path):
     print("case bfs from a CSR file", flush=True)
     row, col = G.rmat_csr(14, 8, 5)
