@@ -754,7 +754,7 @@ def write_spmv(path: str, cols: int, row_ptr, col_idx, val) -> None:
 
 # ---------------------------------------------------------------- sorting
 
-def cilksort(keys, leaf: int = 4096, merge_leaf: int = 32768):
+def cilksort(keys, leaf: int = 4096, merge_leaf: int = 0):
     """Sorted copy of uint32 keys (block-cooperative cilksort on the GPU); returns (keys, stats)."""
     import numpy as np
     a = np.ascontiguousarray(keys, dtype=np.uint32).copy()

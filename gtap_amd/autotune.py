@@ -171,7 +171,7 @@ def workload(name: str, reps: int = 3) -> Tuple[Measure, Dict[str, Sequence[int]
             apply(p)
 
             def one():
-                out, st = gtap_amd.cilksort(keys, leaf=p.get("leaf", 4096), merge_leaf=p.get("merge_leaf", 32768))
+                out, st = gtap_amd.cilksort(keys, leaf=p.get("leaf", 4096), merge_leaf=p.get("merge_leaf", 0))
                 return hash(out.tobytes()), st["kernel_ms"]
             return _median_ms(one, reps)
         return measure, space

@@ -538,22 +538,20 @@ static_assert(CilkProgram::kFrameWords <= 16, "block frame cache holds 16 words"
 
 // Sorts n uint32 keys in place (device buffers keys and tmp, n elements each).
 // leaf <= 4096 keys are sorted by one workgroup in LDS (0 -> 4096; at 4096, ranges of up to 8192
-// are); merges of at most merge_leaf keys are done by one workgroup (0 -> 32768; at most 4096 to
-// 16384 for sorts of up to 32M keys).
+// are); merges of at most merge_leaf keys are done by one workgroup (0 -> 4096 for n up to 2M,
+// 8192 up to 8M, 16384 up to 32M, else 32768).
 // Replaces the program of evaluation/2-comparison/cilksort/gtap_cilksort.cu:169-281.
 extern "C" int gtap_cilksort(uint32_t* keys, uint32_t* tmp, int64_t n, int64_t leaf, int64_t merge_leaf,
                              gtap_run_stats* stats) {
     using namespace gtap;
     if (!keys || !tmp || n < 0) return host::invalid_argument("gtap_cilksort: bad arguments");
     if (leaf <= 0) leaf = 4096;
-    if (merge_leaf <= 0) merge_leaf = 32768;
     if (leaf > cilk::kTile) return host::invalid_argument("gtap_cilksort: leaf must be <= 4096");
-    // A few workgroups merging long runs leave the others idle: with n keys no merge above `most`
-    // stays whole. Measured (us, 4096 / 8192 / 16384 / 32768): 1M keys 418 / 426 / 458 / 550, 4M 635 /
-    // 631 / 671 / 803, 16M 1298 / 1170 / 1169 / 1288, 64M 4424 / 3821 / 3487 / 3340; 20011 keys 139 /
-    // 145 / 147 / 149.
-    const int64_t most = n <= (2 << 20) ? 4096 : (n <= (8 << 20) ? 8192 : (n <= (32 << 20) ? 16384 : merge_leaf));
-    if (merge_leaf > most) merge_leaf = most;
+    // The default by n: a few workgroups merging long runs leave the others idle. Measured (us, 4096 /
+    // 8192 / 16384 / 32768): 1M keys 418 / 426 / 458 / 550, 4M 635 / 631 / 671 / 803, 16M 1298 / 1170 /
+    // 1169 / 1288, 64M 4424 / 3821 / 3487 / 3340; 20011 keys 139 / 145 / 147 / 149. A caller's own
+    // value is taken as it is.
+    if (merge_leaf <= 0) merge_leaf = n <= (2 << 20) ? 4096 : (n <= (8 << 20) ? 8192 : (n <= (32 << 20) ? 16384 : 32768));
     if (merge_leaf < 3) merge_leaf = 3;
     if (n == 0) {
         if (stats) memset(stats, 0, sizeof(*stats));

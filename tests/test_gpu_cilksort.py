@@ -38,6 +38,28 @@ def test_cilksort_cutoffs(leaf, merge_leaf):
         assert np.array_equal(out, oracle.cilksort_u32(keys, leaf, merge_leaf))
 
 
+def sort_nodes(n, leaf):
+    """Ranges of the sort tree above `leaf` keys, each of which spawns 4 sorts and 3 merges."""
+    if n <= leaf:
+        return 0
+    h = n // 2
+    return 1 + sum(sort_nodes(k, leaf) for k in (h // 2, h - h // 2, (n - h) // 2, n - h - (n - h) // 2))
+
+
+@pytest.mark.parametrize("n", [70_003, 200_003, (2 << 20) + 3])
+def test_cilksort_obeys_the_largest_merge(n):
+    """A merge_leaf that the caller gives is taken as it is: with one of n no merge is cut, however
+    many tiles it has; the default cuts them."""
+    print(f"case cilksort merge_leaf of the caller, n={n}", flush=True)
+    keys = oracle.gen_keys_u32(n, n)
+    out, st = gtap_amd.cilksort(keys, leaf=1024, merge_leaf=n)
+    assert np.array_equal(out, np.sort(keys))
+    assert st["tasks_spawned"] == 7 * sort_nodes(n, 1024)
+    out, st = gtap_amd.cilksort(keys, leaf=1024)
+    assert np.array_equal(out, np.sort(keys))
+    assert st["tasks_spawned"] > 7 * sort_nodes(n, 1024)
+
+
 def test_cilksort_benchmark_keys():
     n = 1 << 26
     print(f"case cilksort benchmark n={n}", flush=True)
