@@ -159,7 +159,7 @@ def bench_cilksort(gtap_amd, roofline, hbm_meas, reps: int = 3) -> dict:
     import ctypes
     import numpy as np
     tuned = use_tuned("cilksort")
-    leaf, merge_leaf = int(tuned.get("leaf", 4096)), int(tuned.get("merge_leaf", 0))
+    leaf, merge_leaf = int(tuned.get("leaf", 0)), int(tuned.get("merge_leaf", 0))
     n = 1 << 26
     keys = gtap_amd.gen_keys(n)
     src = gtap_amd.DeviceBuffer.from_array(keys)

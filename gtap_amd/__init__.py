@@ -754,8 +754,9 @@ def write_spmv(path: str, cols: int, row_ptr, col_idx, val) -> None:
 
 # ---------------------------------------------------------------- sorting
 
-def cilksort(keys, leaf: int = 4096, merge_leaf: int = 0):
-    """Sorted copy of uint32 keys (block-cooperative cilksort on the GPU); returns (keys, stats)."""
+def cilksort(keys, leaf: int = 0, merge_leaf: int = 0):
+    """Sorted copy of uint32 keys (block-cooperative cilksort on the GPU; 0: the library's leaf and
+    merge sizes); returns (keys, stats)."""
     import numpy as np
     a = np.ascontiguousarray(keys, dtype=np.uint32).copy()
     s = RunStats()

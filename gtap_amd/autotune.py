@@ -164,14 +164,14 @@ def workload(name: str, reps: int = 3) -> Tuple[Measure, Dict[str, Sequence[int]
     if name == "cilksort":
         import numpy as np
         keys = gtap_amd.gen_keys(1 << 26, 123456789)
-        space = {"block_workers": (0, 256, 512, 768), "merge_leaf": (32768, 16384, 65536, 131072),
-                 "leaf": (4096, 2048, 1024)}
+        space = {"block_workers": (0, 256, 512, 768), "merge_leaf": (0, 16384, 32768, 65536, 131072),
+                 "leaf": (0, 4096, 2048, 1024)}  # 0: the library's own sizes
 
         def measure(p):
             apply(p)
 
             def one():
-                out, st = gtap_amd.cilksort(keys, leaf=p.get("leaf", 4096), merge_leaf=p.get("merge_leaf", 0))
+                out, st = gtap_amd.cilksort(keys, leaf=p.get("leaf", 0), merge_leaf=p.get("merge_leaf", 0))
                 return hash(out.tobytes()), st["kernel_ms"]
             return _median_ms(one, reps)
         return measure, space

@@ -154,8 +154,8 @@ int gtap_bfs_host(const int32_t* row, const int32_t* col, int32_t nv, int64_t ne
                   int32_t* depth_out, int32_t num_queues, int32_t split, gtap_run_stats* stats);
 
 /* Cilksort of n uint32 keys in place, block-cooperative (one task per 256-thread
- * workgroup): keys and tmp are device buffers of n keys; leaves of <= leaf keys (0 -> 4096,
- * max 4096; at 4096, ranges of up to 8192 keys are) are sorted in LDS by one workgroup; merges of
+ * workgroup): keys and tmp are device buffers of n keys; leaves of <= leaf keys (at most
+ * 4096; 0 -> 8192) are sorted in LDS by one workgroup; merges of
  * <= merge_leaf keys (0 -> 4096 for n <= 2M, 8192 for n <= 8M, 16384 for n <= 32M, else 32768) are
  * merged by one workgroup. Replaces evaluation/2-comparison/cilksort/gtap_cilksort.cu:89-281. */
 int gtap_cilksort(uint32_t* keys, uint32_t* tmp, int64_t n, int64_t leaf, int64_t merge_leaf,

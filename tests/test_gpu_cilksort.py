@@ -91,3 +91,25 @@ def test_cilksort_size_rules(n):
     keys = np.random.default_rng(n).integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)
     out, _ = gtap_amd.cilksort(keys)
     assert np.array_equal(out, np.sort(keys))
+
+
+@pytest.mark.parametrize("n", [256, 2049, 4096, 4097, 8191, 8192, 8193, 16385, 32769, 40_000])
+@pytest.mark.parametrize("leaf", [0, 4096, 4095, 2048])
+def test_cilksort_obeys_the_leaf(n, leaf):
+    """A leaf that the caller gives is taken as it is, 4096 too; the default sorts ranges of up to 8192
+    keys whole. (merge_leaf = n: no merge is cut, so the spawns are those of the sort tree.)"""
+    print(f"case cilksort leaf of the caller, n={n} leaf={leaf}", flush=True)
+    rng = np.random.default_rng(n + leaf)
+    for keys in (rng.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32),
+                 np.where(rng.random(n) < 0.5, 0xFFFFFFFF, 0).astype(np.uint32),
+                 np.arange(n, dtype=np.uint32)[::-1].copy(),
+                 rng.integers(0, 3, n).astype(np.uint32)):
+        out, st = gtap_amd.cilksort(keys, leaf=leaf, merge_leaf=n)
+        assert np.array_equal(out, np.sort(keys))
+        assert st["tasks_spawned"] == 7 * sort_nodes(n, leaf or 8192)
+
+
+def test_cilksort_refuses_larger_leaves():
+    print("case cilksort leaf=4097 (refused)", flush=True)
+    with pytest.raises(gtap_amd.GtapError):
+        gtap_amd.cilksort(np.arange(10, dtype=np.uint32), leaf=4097)
