@@ -73,14 +73,14 @@ struct Segment {   // one task's edges in the flat sequence of a round's edges
     int32_t shift; // flat edge f is column entry f + shift
     int32_t nd;    // depth its neighbours get
 };
-struct Hit {
-    int32_t u;
-    int32_t nd;
-};
+// With 4 queues a workgroup takes 50784 bytes of LDS in all; three fit a CU up to 53760 (R-MAT 22
+// with 53856 bytes, two a CU: 1343 us, with three 1161 us).
 struct ExpandShared {
     uint32_t starts[2 * kWindows];  // per window of 64 flat edges, which of them start a segment
     Segment seg[kWave];
-    Hit hit[kHits];
+    uint32_t task[kWave];           // per segment, its task's id, for error reports
+    int32_t hit[kHits];             // improved vertices
+    uint8_t from[kHits];            // the segment that improved them
 };
 
 template <int NQ>
@@ -142,12 +142,13 @@ __device__ __forceinline__ void spawn_hits(T& t, const BfsArgs& g, ExpandShared*
     wave_sync();
     for (int32_t b = 0; b < count; b += kWave) {
         if (b + l < count) {
-            const int32_t u = lds(sh->hit)[b + l].u, nd = lds(sh->hit)[b + l].nd;
+            const int32_t u = lds(sh->hit)[b + l];
+            const uint32_t sg = lds(sh->from)[b + l];
             const int32_t us = g.row[u], ue = g.row[u + 1];
             if (us < 0 || ue < us || (int64_t)ue > g.ne)  // malformed offsets: never read past col
-                GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, u, g.nv);
+                GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, lds(sh->task)[sg], -1, u, g.nv);
             else if (ue > us)
-                spawn_one(t, F_BFS, route<NQ>(ue - us), BfsArg{u, us, ue, nd});
+                spawn_one(t, F_BFS, route<NQ>(ue - us), BfsArg{u, us, ue, lds(sh->seg)[sg].nd});
         }
     }
     wave_sync();
@@ -181,6 +182,7 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
     if (has) {
         lds(sh->seg)[rank_in(hm)].shift = begin - start;
         lds(sh->seg)[rank_in(hm)].nd = nd_own;
+        lds(sh->task)[rank_in(hm)] = t.tid;
     }
     int32_t hits = 0;
     for (int32_t b = 0; b < total; b += kWindows * kWave) {
@@ -192,6 +194,7 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
         wave_sync();
         int32_t before = popc(ballot(has && start < b));  // segments that start before the window
         int32_t u[kWindows], nd[kWindows];
+        uint32_t from[kWindows / 4] = {};  // each edge's segment, 8 bits
 #pragma unroll
         for (int j = 0; j < kWindows; ++j) {
             const uint64_t m = uniform((uint64_t)lds(sh->starts)[2 * j] | ((uint64_t)lds(sh->starts)[2 * j + 1] << 32));
@@ -199,20 +202,23 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
             before += popc(m);
             const int32_t f = b + j * kWave + l;
             const bool in = f < total;
-            const int32_t shift = lds(sh->seg)[in ? r : 0].shift;
-            nd[j] = lds(sh->seg)[in ? r : 0].nd;
+            const uint32_t sg = in ? (uint32_t)r : 0u;
+            const int32_t shift = lds(sh->seg)[sg].shift;
+            nd[j] = lds(sh->seg)[sg].nd;
+            from[j / 4] |= sg << (8 * (j % 4));
             u[j] = in ? g.col[f + shift] : -1;
         }
         bool bad = false;
+        uint32_t bad_from = 0;
 #pragma unroll
         for (int j = 0; j < kWindows; ++j) {
             if (u[j] >= g.nv || u[j] < -1) {
                 bad = true;
-                u[j] = -1;
+                bad_from = from[j / 4] >> (8 * (j % 4)) & 255u;
             }
         }
         if (ballot(bad)) {
-            if (bad) GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, -1, g.nv);
+            if (bad) GTAP_DEVICE_ERROR(*t.dev, GTAP_ERROR_INVALID_ARGUMENT, lds(sh->task)[bad_from], -1, -1, g.nv);
             break;
         }
         int32_t old[kWindows];
@@ -233,8 +239,8 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
                 hits = 0;
             }
             if (hit) {
-                lds(sh->hit)[hits + rank_in(m)].u = u[j];
-                lds(sh->hit)[hits + rank_in(m)].nd = nd[j];
+                lds(sh->hit)[hits + rank_in(m)] = u[j];
+                lds(sh->from)[hits + rank_in(m)] = (uint8_t)(from[j / 4] >> (8 * (j % 4)));
             }
             hits += popc(m);
         }

@@ -1,6 +1,8 @@
 """Asynchronous BFS (EPAQ by out-degree bucket, and one queue) through the C ABI on the
 GPU: distances bit-exact against the oracle's queue BFS, plus the BFS invariants checked
 directly at the benchmark scale."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -124,6 +126,39 @@ def test_bfs_bad_column_in_a_hub_is_reported(queues):
     assert "INVALID_ARGUMENT" in str(e.value)
     depth, st = gtap_amd.bfs(row, col, 0, num_queues=queues)
     assert st["error_code"] == 0 and np.array_equal(depth, oracle.bfs(row, col, 0))
+
+
+@pytest.mark.parametrize("queues", [1, 4])
+@pytest.mark.parametrize("deg", [3, 40, 1000])
+def test_bfs_error_reports_name_the_task(queues, deg):
+    """A bad column and a vertex with malformed offsets are reported with the task that met them
+    (and the vertex), from lane tasks and, with 4 queues and 1000 edges, from a wave task."""
+    print(f"case bfs error reports queues={queues} deg={deg}", flush=True)
+    row, col = hub_graph(deg, extra=0)
+    nv = row.size - 1
+
+    def run(row, col):
+        bufs = [gtap_amd.DeviceBuffer.from_array(a) for a in (row, col, np.zeros(nv, np.int32))]
+        s = gtap_amd.RunStats()
+        st = gtap_amd.lib().gtap_bfs(bufs[0].ptr, bufs[1].ptr, nv, col.size, 0, bufs[2].ptr, queues, 64, ctypes.byref(s))
+        r = gtap_amd.ErrorReport()
+        assert gtap_amd.lib().gtap_get_runtime_error_report(ctypes.byref(r)) == 0
+        for b in bufs:
+            b.free()
+        return st, s.error_code, r
+
+    bad = col.copy()
+    bad[deg // 2] = nv + 5
+    st, code, r = run(row, bad)
+    assert st != 0 and code == 11 and r.valid == 1
+    assert r.tid > 0 and r.limit == nv and r.value == -1
+    bad = row.copy()
+    u = deg // 2 + 1  # a neighbour of the source
+    bad[u + 1] = bad[u] - 1
+    st, code, r = run(bad, col)
+    assert st != 0 and code == 11 and r.valid == 1
+    assert r.tid > 0 and r.limit == nv and r.value in (u, u + 1)
+    assert run(row, col)[0] == 0
 
 
 @pytest.mark.parametrize("degrees", [[1] * 200, [63] * 70, [64] * 70, [65] * 70, [0, 7, 0, 64, 1, 0, 511, 3] * 30,
