@@ -18,7 +18,7 @@ struct Steps {
     uint32_t n, step, at;
     GTAP_STEPS_FN bool on() const { return at < n; }                        // items are left
     GTAP_STEPS_FN uint32_t left() const { return at < n ? n - at : 0u; }  // how many, this step's included
-    GTAP_STEPS_FN bool more() const { return left() > step; }               // a further step is needed
+    GTAP_STEPS_FN bool more() const { return at + step < n; }               // a further step is needed
     GTAP_STEPS_FN void next() { at += step; }
     // How many steps the walk takes. A loop that counts them is one whose length the compiler
     // knows and unrolls, which it does not for positions that may wrap (tree of height 15: 219 us

@@ -219,14 +219,15 @@ __device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveSh
 #pragma unroll
         for (int j = 0; j < kPer; ++j) tile[slot * stride + j * g + sub] = Entry{v[j], xv[j]};
         wave_sync();
-        const uint32_t left = add.left();
-        for (uint32_t e = 0; e < add.step && e < left; e += kPer) {
+        // signed, so that the tile's addresses fold into one base (200003 rows of 100: 313 against 326 us)
+        const int32_t left = (int32_t)(add.more() ? add.step : add.left());
+        for (int32_t e = 0; e < left; e += kPer) {
             Entry t[kPer];
 #pragma unroll
-            for (int j = 0; j < kPer; ++j) t[j] = tile[l * stride + (int32_t)e + j];
+            for (int j = 0; j < kPer; ++j) t[j] = tile[l * stride + e + j];
 #pragma unroll
             for (int j = 0; j < kPer; ++j)
-                if (e + (uint32_t)j < left) sum = __builtin_fma(t[j].x, t[j].y, sum);
+                if (e + j < left) sum = __builtin_fma(t[j].x, t[j].y, sum);
         }
         add.next();
         if (!more) {
