@@ -207,7 +207,11 @@ __device__ __forceinline__ void Program::run_coop(L& lane, uint64_t mask, WaveSh
             bad |= in && !valid;
             xv[j] = in && valid ? a.x[c[j]] : 0.0;
         }
-        if (bad) GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, -1, -1, begin, a.cols);
+        if (ballot(bad)) {
+            const int32_t src = lds(sh->src)[p0 + slot < m ? p0 + slot : 0];
+            const int32_t bad_row = shfl((int32_t)lane.frame[0], src), bad_task = shfl((int32_t)lane.tid, src);
+            if (bad) GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, bad_task, -1, bad_row, a.cols);
+        }
         const bool more = ballot(load.more()) != 0;
         load.at = more ? load.at + load.step : 0u;
         const int32_t p1 = more ? p0 : p0 + rows;

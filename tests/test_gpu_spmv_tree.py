@@ -89,6 +89,22 @@ def test_spmv_bad_column_is_reported():
     assert np.array_equal(G.spmv(rp, ci, va, np.ones(500))[0], O.spmv(rp, ci, va, np.ones(500)))
 
 
+@pytest.mark.parametrize("avg,row,at", [(3, 0, 0), (3, 399, 1), (30, 250, 20), (200, 77, 0), (200, 300, 150), (900, 2, 700)])
+def test_spmv_bad_column_report_names_task_and_row(avg, row, at):
+    """Rows of 1 to 64 lanes and of several steps; the entry's offset is not the row."""
+    print(f"case spmv bad column report avg={avg} row={row} at={at}", flush=True)
+    n = 400
+    lengths = np.full(n, avg)
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    ci = np.tile(np.arange(avg, dtype=np.int32), n)
+    ci[rp[row] + at] = 1000
+    with pytest.raises(G.GtapError) as e:
+        G.spmv(rp, ci, np.ones(ci.size), np.ones(1000), 1000)
+    r = e.value.report
+    assert e.value.code == 11 and r["valid"] == 1
+    assert r["value"] == row and r["limit"] == 1000 and r["tid"] > 0
+
+
 @pytest.mark.parametrize("height,mem_ops,iters", [(0, 4, 4), (1, 0, 0), (5, 64, 512), (10, 16, 32), (15, 64, 512),
                                                   (12, 0, 1000)])
 def test_tree_matches_oracle(height, mem_ops, iters):
