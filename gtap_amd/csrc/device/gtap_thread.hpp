@@ -1108,7 +1108,7 @@ __device__ __forceinline__ bool window_append(const GtapDev& dev, WaveCtxOf<P>* 
     const uint32_t cnt = (uint32_t)popc(m), r = (uint32_t)rank_in(m);
     if (tail + cnt - dtop > dev.cap - kMargin) dtop = uniform((uint32_t)(ld64(dq_word_ptr(dev, q, me)) >> 32));
     if (tail + cnt - dtop > dev.cap - kMargin) {
-        if (lane_id() == 0) GTAP_DEVICE_ERROR(dev, GTAP_ERROR_QUEUE_OVERFLOW, -1, q, tail + cnt - dtop, dev.cap - kMargin);
+        if (mine && r == 0) GTAP_DEVICE_ERROR(dev, GTAP_ERROR_QUEUE_OVERFLOW, id, q, tail + cnt - dtop, dev.cap - kMargin);
         return false;
     }
     const uint32_t slot = (tail + r) & (kWave - 1);

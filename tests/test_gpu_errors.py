@@ -70,6 +70,23 @@ def test_joined_children_beyond_deque_capacity(mods):
     clean_chain(m)
 
 
+def test_resumed_parents_beyond_deque_capacity(mods):
+    """64 parents that resume together after their round's spawns have nearly filled the deque: the
+    queue overflow (3) names the first of them."""
+    m = gtap_amd.EntryModule(gbuild.lowered_lib("crowd"), "crowd")
+    for n, code in ((20000, 0), (31700, 3), (20000, 0)):
+        print(f"case crowd({n}) (error {code} expected)", flush=True)
+        m.set_symbol("d_out", -1, ctypes.c_longlong)
+        assert m.launch("crowd_kernel", [I], n, grid=1) == 0
+        assert gtap_amd.gtap_get_runtime_error_code() == code
+        if code:
+            r = report()
+            assert r.valid == 1 and r.code == 3 and r.queue_idx == 0
+            assert r.value == n + 64 and r.limit == 32768 - 1024 and r.tid > 0
+        else:
+            assert m.get_symbol("d_out", ctypes.c_longlong) == 64
+
+
 def test_joined_child_left_behind(mods):
     print("case task returning before its taskwait (error 8 expected)", flush=True)
     m = mods["errors"]
