@@ -67,6 +67,7 @@ __host__ __device__ __forceinline__ uint32_t degree_bucket(int32_t deg) {
 constexpr int32_t kSplitFanout = 8;         // pieces per split of a lane task's range
 constexpr int32_t kWaveSplitEdges = 2048;  // a wave task scans at most this many edges (and cap / 8)
 constexpr int kWindows = 8;                 // edges per lane per step of an expansion
+constexpr int32_t kMaxExpand = 1 << 20;     // edges of one range in one scan: 64 of them stay within an int32
 constexpr int kHits = 192;                  // improved vertices held before their tasks are spawned
 
 struct Segment {   // one task's edges in the flat sequence of a round's edges
@@ -256,7 +257,7 @@ __device__ __forceinline__ void Program<NQ>::run(L& lane) {
     const int32_t s = lane.template arg<int32_t>(4);
     const int32_t e = lane.template arg<int32_t>(8);
     const int32_t d = lane.template arg<int32_t>(12);
-    // stale: v was reached by a shorter path meanwhile
+    // else v was reached by a shorter path meanwhile
     if (ld32(reinterpret_cast<const int32_t*>(g.depth) + v) >= d) {
         if (e - s > g.split) {
             // up to kSplitFanout near-equal pieces, each routed by its own length
@@ -279,8 +280,14 @@ template <int NQ>
 template <class L>
 __device__ __forceinline__ void Program<NQ>::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
     (void)mask;
-    const int32_t s = (int32_t)lane.frame[1], e = (int32_t)lane.frame[2];
-    expand<NQ>(lane, *lane.args, sh, s, lane.coop ? e - s : 0, (int32_t)lane.frame[3] + 1);
+    const int32_t s = (int32_t)lane.frame[1], nd = (int32_t)lane.frame[3] + 1;
+    int32_t left = lane.coop ? (int32_t)lane.frame[2] - s : 0, at = s;
+    do {
+        const int32_t n = left < kMaxExpand ? left : kMaxExpand;
+        expand<NQ>(lane, *lane.args, sh, at, n, nd);
+        at += n;
+        left -= n;
+    } while (NQ == 1 && ballot(left > 0));  // again with splits above kMaxExpand only
 }
 
 // The wave form of the same task (queue 3 with 4 queues): all 64 lanes enter with one (v, s, e, d).
@@ -386,8 +393,6 @@ using Bfs4 = gtap::bfs::Program<4>;
 
 namespace {
 
-constexpr int32_t kMaxSplit = 1 << 20;   // 64 ranges of a round stay within 32-bit edge counts
-
 __global__ void bfs_init_depth(int32_t* depth, int32_t nv, int32_t source) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -407,7 +412,6 @@ extern "C" int gtap_bfs(const int32_t* row, const int32_t* col, int32_t nv, int6
         return host::invalid_argument("gtap_bfs: bad graph arguments");
     if (num_queues != 1 && num_queues != 4) return host::invalid_argument("gtap_bfs: num_queues must be 1 or 4");
     if (split <= 0) split = 64;
-    if (split > kMaxSplit) split = kMaxSplit;
     host::Runtime& R = host::rt();
     if (!R.initialized) {
         int st = gtap_initialize();

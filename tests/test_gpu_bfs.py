@@ -181,6 +181,20 @@ def test_bfs_flat_edge_windows(degrees, queues, split):
     assert np.array_equal(depth, oracle.bfs(row, col, 0))
 
 
+def test_bfs_obeys_a_large_split():
+    """A split of the caller's is taken as it is: with 2^30 a range of more than 2^20 edges is one
+    task (the columns repeat, so its 100 neighbours, without out-edges, are all there is to find)."""
+    deg = (1 << 20) + 77
+    row = np.full(102, deg, np.int32)
+    row[0] = 0
+    col = np.tile(np.arange(1, 101, dtype=np.int32), deg // 100 + 1)[:deg]
+    for split, tasks in ((1 << 30, 1), (1 << 20, 3)):
+        print(f"case bfs split={split}", flush=True)
+        depth, st = gtap_amd.bfs(row, col, 0, num_queues=1, split=split)
+        assert depth[0] == 0 and np.all(depth[1:] == 1)
+        assert st["tasks_executed"] == tasks
+
+
 def test_bfs_split_thresholds_agree():
     row, col = oracle.rmat_csr(13, 16, 11)
     ref = oracle.bfs(row, col, 0)
