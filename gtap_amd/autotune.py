@@ -32,7 +32,7 @@ CONFIG_KEYS = ("blocks", "block_workers", "probe_lanes", "steal_batch", "deque_c
 # The first value of each coordinate is the runtime's default and the search's start point.
 DEFAULT_SPACE: Dict[str, Sequence[int]] = {
     "blocks": (0, 256, 512, 1024, 1536),
-    "probe_lanes": (8, 1, 4, 16, 32),
+    "probe_lanes": (0, 1, 4, 8, 16, 32),
     "steal_batch": (64, 8, 16, 32),
     "deque_capacity": (32768, 65536),
     "xcd_steal": (0, 1),

@@ -118,7 +118,7 @@ struct GtapDev {
     uint32_t ovf_cap;          // cells per overflow ring (power of two)
     uint32_t epaq_publish;     // 1: non-batch EPAQ queues publish their whole private window each round
     uint32_t xcd_steal;        // 1: even probe lanes pick victims on the thief's XCD
-    uint32_t xcd_pad;
+    uint32_t probes_set;       // 1: the caller chose probe_lanes, which idle waves keep to as well
 };
 
 // Round phases of the thread-mode loop, timed in the profiling build with the shader clock

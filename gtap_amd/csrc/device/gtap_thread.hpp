@@ -93,7 +93,8 @@ struct HasLaneSum<P, decltype((void)P::kLaneSum)> {
 };
 
 // Victims an idle wave probes per steal attempt once kPatientAfter attempts in a row have found
-// nothing: all of gtap_config.probe_lanes, or P::kIdleProbes if that is fewer. At launch start and
+// nothing: all of gtap_config.probe_lanes, or P::kIdleProbes if that is fewer and the caller left
+// probe_lanes at its default (one that the caller sets is kept to). At launch start and
 // end thousands of waves are idle, and 8 lines each every 1.3 us is nearly half of the random
 // reads the memory serves; programs whose rounds are bound by memory run faster with 2, those of
 // short dependent rounds find work later with fewer than 8. Measured with 8 / 2 (us): R-MAT 18
@@ -1809,8 +1810,8 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
                 st.jobs += n;
                 batch_q = -1;
             }
-            const uint32_t nprobe = idle_iter >= kPatientAfter && IdleProbes<P>::value < dev.probe_lanes
-                                        ? IdleProbes<P>::value : dev.probe_lanes;
+            const bool fewer = idle_iter >= kPatientAfter && !dev.probes_set && IdleProbes<P>::value < dev.probe_lanes;
+            const uint32_t nprobe = fewer ? IdleProbes<P>::value : dev.probe_lanes;
             if (n == 0) {
                 if constexpr (kStealAnyQueue && Sched == kSchedWS && Q > 1) {
                     uint32_t sq = 0;

@@ -110,7 +110,8 @@ typedef struct gtap_config {
     uint32_t num_queues;      /* EPAQ queues provisioned (default 4) */
     uint32_t blocks;          /* workgroups per launch (default: all co-resident) */
     uint32_t steal_batch;     /* max tasks per steal, <= 64 (default 64) */
-    uint32_t probe_lanes;     /* victims probed per steal attempt, <= 64 (default 8) */
+    uint32_t probe_lanes;     /* victims probed per steal attempt, <= 64 (default 8; by default SpMV,
+                                 n-queens with a cutoff and BFS probe 2 after 8 failed attempts) */
     uint32_t max_jobs;        /* job table / anchor capacity (default 65536) */
     uint32_t timeout_ms;      /* device watchdog (default 20000) */
     uint32_t block_workers;   /* workgroups of the block-mode scheduler (default: co-resident) */

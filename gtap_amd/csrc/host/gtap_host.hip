@@ -150,6 +150,7 @@ GtapDev make_dev(uint32_t nworkers, uint32_t term_mode, uint32_t njobs, gtap_job
     d.ovf_epoch = R.ovf_epoch;
     d.epaq_publish = R.cfg.epaq_publish ? 1u : 0u;
     d.xcd_steal = R.cfg.xcd_steal ? 1u : 0u;
+    d.probes_set = R.probes_set ? 1u : 0u;
     d.idle_level = 1;
     for (uint32_t v = R.cfg.idle_sleep; v > 1 && d.idle_level < 6; v >>= 1) d.idle_level += 1;
     d.prof_having = R.prof_having;
@@ -407,9 +408,11 @@ static void free_all() {
     if (R.ev0) (void)hipEventDestroy(R.ev0);
     if (R.ev1) (void)hipEventDestroy(R.ev1);
     if (R.stream) (void)hipStreamDestroy(R.stream);
-    gtap_config keep = R.cfg;
+    const gtap_config keep = R.cfg;
+    const bool probes_set = R.probes_set;
     R = Runtime();
     R.cfg = keep;
+    R.probes_set = probes_set;
 }
 
 // Lowered modules whose entry kernels the host launches (gtap_register_entry_module).
@@ -470,6 +473,7 @@ int gtap_set_config(const gtap_config* cfg) {
     if (cfg && cfg->xcd_steal > 1) return invalid_argument("gtap_config.xcd_steal must be 0 or 1");
     if (cfg) R.cfg = *cfg;
     else memset(&R.cfg, 0, sizeof(R.cfg));
+    R.probes_set = R.cfg.probe_lanes >= 1 && R.cfg.probe_lanes <= 64;  // anything else: the default
     return 0;
 }
 

@@ -44,6 +44,7 @@ struct Runtime {
     bool initialized = false;
     int device = 0;
     gtap_config cfg{};
+    bool probes_set = false;           // the caller's gtap_config named probe_lanes
     int num_cus = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

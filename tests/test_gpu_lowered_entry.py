@@ -139,6 +139,41 @@ def test_second_launch_needs_a_reset(mods):
     assert m.get_symbol("d_fib_result", ctypes.c_longlong) == 144
 
 
+SETUP = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64)
+_probes_set = []
+
+
+@SETUP
+def _see_descriptor(desc, nbytes):
+    _probes_set.append(ctypes.c_uint32.from_address(desc + nbytes - 4).value)  # GtapDev::probes_set, the last word
+    return 0
+
+
+def test_configured_probe_lanes_are_kept_to(mods):
+    """Launches know whether the caller named probe_lanes: idle waves of some programs probe fewer
+    victims only if not. What was configured outlives gtap_finalize; 0 and values out of range are the
+    default."""
+    stride = gtap_amd.gtap_get_config()["record_stride"]
+    gtap_amd._check(gtap_amd.lib().gtap_register_entry_module(_see_descriptor), "gtap_register_entry_module")
+    try:
+        for probes, expect in ((8, 1), (0, 0), (16, 1), (65, 0), (None, 0)):
+            print(f"case probe_lanes={probes}", flush=True)
+            assert gtap_amd.gtap_finalize() == 0
+            cfg = {} if probes is None else {"probe_lanes": probes}
+            assert gtap_amd.gtap_set_config(timeout_ms=20000, record_stride=stride, **cfg) == 0
+            for again in (False, True):
+                _probes_set.clear()
+                assert gtap_amd.gtap_initialize() == 0
+                assert _probes_set == [expect]
+                v, _ = gtap_amd.nqueens_cutoff(9, 4)
+                assert v == 352
+                assert gtap_amd.gtap_finalize() == 0
+    finally:
+        gtap_amd.gtap_finalize()
+        gtap_amd.gtap_set_config(timeout_ms=20000, record_stride=stride)
+        assert gtap_amd.gtap_initialize() == 0
+
+
 def test_launch_with_a_smaller_grid(mods):
     """Any grid of 256-thread workgroups runs the program (fewer workers than co-resident)."""
     print("case fib on 3 workgroups", flush=True)
