@@ -37,6 +37,8 @@
 // lane tasks and their split tasks. One queue keeps the lane program for every range. (The
 // reference cuts a long list into 32-edge tasks all spawned by one task,
 // asynchronous_bfs_thread.cu:25-33; a bounded fan-out keeps one lane's spawn loop short.)
+#include <type_traits>
+
 #include "../device/gtap_abi.hpp"
 #include "../device/gtap_block.hpp"
 #include "../host/gtap_launch.hpp"
@@ -84,7 +86,9 @@ struct ExpandShared {
     uint8_t from[kHits];            // the segment that improved them
 };
 
-template <int NQ>
+// kFlat: the ranges of a round are scanned as one sequence by the whole wave (expand), else one
+// range of at most kShortSplit edges per lane (lane_scan).
+template <int NQ, bool kFlat = true>
 struct Program {
     static constexpr int kQueues = NQ;
     static constexpr int kWaveQueue = NQ == 4 ? 3 : -1;
@@ -95,15 +99,13 @@ struct Program {
     static constexpr uint32_t kMaxFunc = F_BFS;
     static constexpr uint32_t kFrameBytes = 16;
     using Args = BfsArgs;
-    using WaveShared = ExpandShared;
-    static constexpr bool kCoop = true;  // the edges of a round are scanned by run_coop
+    using WaveShared = std::conditional_t<kFlat, ExpandShared, int32_t>;
+    static constexpr bool kCoop = kFlat;  // the edges of a round are scanned by run_coop
     // With one queue a wave holds few tasks while the search spreads, and batches of 32 tasks of up
     // to 64 edges spread it sooner: R-MAT 18, 64 / 32 / 16 a batch: 297 / 258 / 286 us. Ranges cut
     // smaller than that make a batch of 32 too little work for its round (R-MAT 22 in ranges of 32
-    // edges, 32 / 64 a batch: 1212 / 995 us; of 16 edges: 1700 / 1236 us), so a batch holds 2048
-    // edges' worth of tasks. (One range per lane without the flat scan took 1050 and 1152 us there:
-    // ranges of 16 edges are the one size that it scans faster.) With four queues, each queue's
-    // batch is smaller anyway: R-MAT 22, 64 / 32: 1116 / 1196 us.
+    // edges, 32 / 64 a batch: 1212 / 995 us), so a batch holds 2048 edges' worth of tasks. With four
+    // queues, each queue's batch is smaller anyway: R-MAT 22, 64 / 32: 1116 / 1196 us.
     __device__ __forceinline__ static uint32_t batch_cap(const Args& g) {
         if constexpr (NQ != 1) return (uint32_t)kWave;
         const uint32_t n = g.split > 0 ? (uint32_t)(2048 / g.split) : (uint32_t)kWave;
@@ -249,9 +251,52 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
     if (hits) spawn_hits<NQ>(t, g, sh, hits);
 }
 
-template <int NQ>
+// Ranges of up to kShortSplit edges, one per lane: the column loads, the depth probes and the
+// atomics of a range are issued back to back, and its improved vertices spawned one a turn. The
+// flat scan's fixed work per round (prefix sum, window masks, hit list) does not pay for so few
+// edges, and it takes children in an order that expands more vertices twice. One queue, flat / per
+// lane (us): R-MAT 22, split 8: 1590 / 1370, 16: 1245 / 1106, 24: 1080 / 1070, 32: 995 / 1013;
+// R-MAT 20, 16: 415 / 408, 24: 415 / 420; R-MAT 18, 8: 283 / 268, 16: 263 / 254, 24: 249 / 259.
+constexpr int32_t kShortSplit = 16;
+template <int NQ, class L>
+__device__ __forceinline__ void lane_scan(L& lane, const BfsArgs& g, int32_t s, int32_t e, int32_t nd) {
+    int32_t u[kShortSplit], old[kShortSplit];
+#pragma unroll
+    for (int j = 0; j < kShortSplit; ++j) u[j] = s + j < e ? g.col[s + j] : -1;
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < kShortSplit; ++j) bad |= u[j] >= g.nv || u[j] < -1;
+    if (bad) {
+        GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, -1, g.nv);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < kShortSplit; ++j) old[j] = u[j] >= 0 ? g.depth[u[j]] : 0;
+    uint32_t hits = 0;
+#pragma unroll
+    for (int j = 0; j < kShortSplit; ++j) {
+        if (old[j] > nd)
+            old[j] = __hip_atomic_fetch_min(g.depth + u[j], nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int j = 0; j < kShortSplit; ++j) hits |= (old[j] > nd ? 1u : 0u) << j;
+    while (hits) {
+        const int j = __builtin_ctz(hits);
+        hits &= hits - 1u;
+        int32_t v = u[0];
+#pragma unroll
+        for (int k = 1; k < kShortSplit; ++k) v = j == k ? u[k] : v;
+        const int32_t us = g.row[v], ue = g.row[v + 1];
+        if (us < 0 || ue < us || (int64_t)ue > g.ne)  // malformed offsets: never read past col
+            GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, v, g.nv);
+        else
+            spawn_one(lane, F_BFS, route<NQ>(ue - us), BfsArg{v, us, ue, nd});
+    }
+}
+
+template <int NQ, bool kFlat>
 template <class L>
-__device__ __forceinline__ void Program<NQ>::run(L& lane) {
+__device__ __forceinline__ void Program<NQ, kFlat>::run(L& lane) {
     const BfsArgs& g = *lane.args;
     const int32_t v = lane.template arg<int32_t>(0);
     const int32_t s = lane.template arg<int32_t>(4);
@@ -269,16 +314,18 @@ __device__ __forceinline__ void Program<NQ>::run(L& lane) {
                 const int32_t pe = s + (int32_t)(len * (i + 1) / k);
                 __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
             }
-        } else {
+        } else if constexpr (kFlat) {
             lane.coop = true;  // its edges: run_coop
+        } else {
+            lane_scan<NQ>(lane, g, s, e, d + 1);
         }
     }
     __gtap_finish_task(lane);
 }
 
-template <int NQ>
+template <int NQ, bool kFlat>
 template <class L>
-__device__ __forceinline__ void Program<NQ>::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
+__device__ __forceinline__ void Program<NQ, kFlat>::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
     (void)mask;
     const int32_t s = (int32_t)lane.frame[1], nd = (int32_t)lane.frame[3] + 1;
     int32_t left = lane.coop ? (int32_t)lane.frame[2] - s : 0, at = s;
@@ -291,9 +338,9 @@ __device__ __forceinline__ void Program<NQ>::run_coop(L& lane, uint64_t mask, Wa
 }
 
 // The wave form of the same task (queue 3 with 4 queues): all 64 lanes enter with one (v, s, e, d).
-template <int NQ>
+template <int NQ, bool kFlat>
 template <class W>
-__device__ __forceinline__ void Program<NQ>::run_wave(W& wt) {
+__device__ __forceinline__ void Program<NQ, kFlat>::run_wave(W& wt) {
     const BfsArgs& g = *wt.args;
     const int32_t v = wt.template arg<int32_t>(0);
     const int32_t s = wt.template arg<int32_t>(4);
@@ -389,6 +436,7 @@ static_assert(kBlockEdges <= (int32_t)kBlockMaxSpawn, "one invocation spawns at 
 }  // namespace gtap
 
 using Bfs1 = gtap::bfs::Program<1>;
+using Bfs1Short = gtap::bfs::Program<1, false>;
 using Bfs4 = gtap::bfs::Program<4>;
 
 namespace {
@@ -427,6 +475,7 @@ extern "C" int gtap_bfs(const int32_t* row, const int32_t* col, int32_t nv, int6
     gtap_job job = host::make_job(bfs::F_BFS, q, &root, sizeof(root));
     bfs::BfsArgs a{row, col, depth, nv, split, ne};
     if (num_queues == 4) return host::run_single_job<Bfs4>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
+    if (split <= bfs::kShortSplit) return host::run_single_job<Bfs1Short>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
     return host::run_single_job<Bfs1>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
 }
 

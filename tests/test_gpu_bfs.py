@@ -181,6 +181,28 @@ def test_bfs_flat_edge_windows(degrees, queues, split):
     assert np.array_equal(depth, oracle.bfs(row, col, 0))
 
 
+@pytest.mark.parametrize("split", [1, 2, 15, 16, 17])
+@pytest.mark.parametrize("degrees", [[1] * 100, [15, 16, 17, 0, 1] * 30, [32, 33, 128, 129, 0, 1025] * 10])
+def test_bfs_short_splits(degrees, split):
+    """With one queue, ranges of up to 16 edges are scanned one per lane: lists around multiples of
+    the split and of the 8 pieces a range is cut into, and both sides of the rule."""
+    print(f"case bfs short splits degrees={degrees[:6]} split={split}", flush=True)
+    k = len(degrees)
+    rng = np.random.default_rng(k + split)
+    n = 1 + k + 500
+    adj = [np.arange(1, k + 1)] + [rng.integers(0, n, d) for d in degrees]
+    adj += [rng.integers(0, n, rng.integers(0, 3)) for _ in range(n - 1 - k)]
+    row = np.concatenate([[0], np.cumsum([len(a) for a in adj])]).astype(np.int32)
+    col = np.concatenate(adj).astype(np.int32)
+    depth, st = gtap_amd.bfs(row, col, 0, num_queues=1, split=split)
+    assert st["error_code"] == 0
+    assert np.array_equal(depth, oracle.bfs(row, col, 0))
+    col[k // 2] = n + 3
+    with pytest.raises(gtap_amd.GtapError) as e:
+        gtap_amd.bfs(row, col, 0, num_queues=1, split=split)
+    assert e.value.code == 11 and e.value.report["tid"] > 0 and e.value.report["limit"] == n
+
+
 def test_bfs_obeys_a_large_split():
     """A split of the caller's is taken as it is: with 2^30 a range of more than 2^20 edges is one
     task (the columns repeat, so its 100 neighbours, without out-edges, are all there is to find)."""
