@@ -122,6 +122,15 @@ template <class P>
 struct BatchCap<P, decltype((void)&P::batch_cap)> {
     __device__ __forceinline__ static uint32_t of(const typename P::Args& a) { return P::batch_cap(a); }
 };
+// A program may change the wave's cap after each round's run_coop (P::kRoundCap, P::round_cap(lane)).
+template <class P, class = void>
+struct HasRoundCap {
+    static constexpr bool value = false;
+};
+template <class P>
+struct HasRoundCap<P, decltype((void)P::kRoundCap)> {
+    static constexpr bool value = P::kRoundCap;
+};
 
 // Per-wave scheduler state in LDS.
 //
@@ -784,7 +793,7 @@ struct Lane {
     bool sum_join;          // the pending taskwait is an additive join
     uint32_t total;         // this lane's part of the launch's count (HasLaneSum programs)
     bool coop;              // run_coop finishes this task's body (HasCoop programs)
-    uint32_t coop_arg;      // what the body leaves for run_coop
+    uint32_t coop_arg;      // what the body leaves for run_coop (0 at the launch's start)
     int64_t jsum;           // sum of the children's results, after an additive join
     uint64_t join_delta;    // what finishing adds to the parent's join word
     uint32_t frame[FW];     // the first frame words, loaded when the round starts
@@ -1743,8 +1752,9 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
     L.me = me;
     L.rs = pool_rsrc(dev.recs);
     constexpr int QL = CtxShape<P>::kQL;
-    const uint32_t bcap = BatchCap<P>::of(args);
+    uint32_t bcap = BatchCap<P>::of(args);
     if constexpr (HasLaneSum<P>::value) L.total = 0u;
+    if constexpr (HasCoop<P>::value) L.coop_arg = 0u;
 
     uint32_t rng = 0x9E3779B9u ^ (me * 0x85EBCA6Bu) ^ ((uint32_t)lane * 0xC2B2AE35u) ^ (uint32_t)t_begin;
     if (rng == 0) rng = 1;
@@ -1983,6 +1993,7 @@ __device__ __forceinline__ void thread_scheduler(const GtapDev& dev, const typen
         if constexpr (HasCoop<P>::value) {
             const uint64_t cm = ballot(L.coop);
             if (cm) P::run_coop(L, cm, reinterpret_cast<typename WaveSharedOf<P>::type*>(wave_shared));
+            if constexpr (HasRoundCap<P>::value) bcap = P::round_cap(L);
         }
         phase_mark(PH_RUN);
 

@@ -37,6 +37,8 @@
 // lane tasks and their split tasks. One queue keeps the lane program for every range. (The
 // reference cuts a long list into 32-edge tasks all spawned by one task,
 // asynchronous_bfs_thread.cu:25-33; a bounded fan-out keeps one lane's spawn loop short.)
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "../device/gtap_abi.hpp"
@@ -60,6 +62,7 @@ struct BfsArgs {
     int32_t nv;
     int32_t split;
     int64_t ne;  // column entries: a vertex's offsets must satisfy 0 <= row[u] <= row[u+1] <= ne
+    int32_t hub;   // a wave scans its rounds flat once it has met a range longer than this (-1: at once)
 };
 
 __host__ __device__ __forceinline__ uint32_t degree_bucket(int32_t deg) {
@@ -86,8 +89,8 @@ struct ExpandShared {
     uint8_t from[kHits];            // the segment that improved them
 };
 
-// kFlat: the ranges of a round are scanned as one sequence by the whole wave (expand), else one
-// range of at most kShortSplit edges per lane (lane_scan).
+// kFlat: the ranges of a round are scanned as one sequence by the whole wave (expand), from the
+// start or once the wave has met a hub; else, and until then, one range per lane (lane_scan).
 template <int NQ, bool kFlat = true>
 struct Program {
     static constexpr int kQueues = NQ;
@@ -110,6 +113,16 @@ struct Program {
         if constexpr (NQ != 1) return (uint32_t)kWave;
         const uint32_t n = g.split > 0 ? (uint32_t)(2048 / g.split) : (uint32_t)kWave;
         return n < 32u ? 32u : (n > (uint32_t)kWave ? (uint32_t)kWave : n);
+    }
+    // A wave that has not met a hub takes full batches: with 32 a search of a large graph without
+    // hubs goes deeper first and expands more vertices twice (4M vertices of 4 edges, 32 / 64 a
+    // batch: 16.9 / 10.7 M tasks, 2350 / 1550 us).
+    static constexpr bool kRoundCap = kFlat;
+    template <class L>
+    __device__ __forceinline__ static uint32_t round_cap(L& lane) {
+        const bool met = ballot(lane.coop_arg) != 0ull;
+        lane.coop_arg = met;  // on every lane: the next round may leave the lane that met it without a task
+        return met ? batch_cap(*lane.args) : (uint32_t)kWave;
     }
     template <class L>
     __device__ __forceinline__ static void run(L& lane);
@@ -251,41 +264,54 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
     if (hits) spawn_hits<NQ>(t, g, sh, hits);
 }
 
-// Ranges of up to kShortSplit edges, one per lane: the column loads, the depth probes and the
-// atomics of a range are issued back to back, and its improved vertices spawned one a turn. The
-// flat scan's fixed work per round (prefix sum, window masks, hit list) does not pay for so few
-// edges, and it takes children in an order that expands more vertices twice. One queue, flat / per
-// lane (us): R-MAT 22, split 8: 1590 / 1370, 16: 1245 / 1106, 24: 1080 / 1070, 32: 995 / 1013;
-// R-MAT 20, 16: 415 / 408, 24: 415 / 420; R-MAT 18, 8: 283 / 268, 16: 263 / 254, 24: 249 / 259.
+// One range of up to kLaneEdges edges per lane: the column loads, the depth probes and the atomics
+// of a range are issued back to back, and its improved vertices spawned one a turn. Where it is
+// the better form:
+// - splits of up to kShortSplit edges with one queue. The flat scan's fixed work per round (prefix
+//   sum, window masks, hit list) does not pay for so few edges. Flat / per lane (us): R-MAT 22,
+//   split 8: 1590 / 1370, 16: 1245 / 1106, 24: 1080 / 1070, 32: 995 / 1013; R-MAT 20, 16: 415 / 408,
+//   24: 415 / 420; R-MAT 18, 8: 283 / 268, 16: 263 / 254, 24: 249 / 259;
+// - large graphs without hubs, where the flat scan's rounds of equal ranges gain nothing and its
+//   search expands more vertices twice. Uniform random graphs of 4M vertices and 4 / 8 / 16 edges a
+//   vertex, flat with batches of 32 / per lane (us): one queue 2350 / 1455, 3180 / 1910, 3610 / 2440;
+//   four queues (batches of 64) 1548 / 1438, 2200 / 1830, 3600 / 2430; 1M vertices of 16 edges 484 /
+//   473 and 648 / 487. A graph is large here above 2^19 vertices (400K vertices with 16 edges a
+//   vertex, their ends drawn at random: flat 325, per lane 384 us) and, with four queues, of at
+//   least 8 edges a vertex (1M vertices of 4 drawn edges: 546 / 700 us). R-MAT graphs have hubs:
+//   their waves turn to the flat scan within a round or two and keep its gain.
 constexpr int32_t kShortSplit = 16;
+template <int NQ>
+constexpr int32_t kLaneEdges = NQ == 4 ? 8 : kShortSplit;  // with four queues 16 spill 20 registers, 8 spill 7
+static_assert(kLaneEdges<1> >= kShortSplit, "a short range is scanned at once");
 template <int NQ, class L>
 __device__ __forceinline__ void lane_scan(L& lane, const BfsArgs& g, int32_t s, int32_t e, int32_t nd) {
-    int32_t u[kShortSplit], old[kShortSplit];
+    constexpr int32_t kC = kLaneEdges<NQ>;
+    int32_t u[kC], old[kC];
 #pragma unroll
-    for (int j = 0; j < kShortSplit; ++j) u[j] = s + j < e ? g.col[s + j] : -1;
+    for (int j = 0; j < kC; ++j) u[j] = s + j < e ? g.col[s + j] : -1;
     bool bad = false;
 #pragma unroll
-    for (int j = 0; j < kShortSplit; ++j) bad |= u[j] >= g.nv || u[j] < -1;
+    for (int j = 0; j < kC; ++j) bad |= u[j] >= g.nv || u[j] < -1;
     if (bad) {
         GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, -1, g.nv);
         return;
     }
 #pragma unroll
-    for (int j = 0; j < kShortSplit; ++j) old[j] = u[j] >= 0 ? g.depth[u[j]] : 0;
+    for (int j = 0; j < kC; ++j) old[j] = u[j] >= 0 ? g.depth[u[j]] : 0;
     uint32_t hits = 0;
 #pragma unroll
-    for (int j = 0; j < kShortSplit; ++j) {
+    for (int j = 0; j < kC; ++j) {
         if (old[j] > nd)
             old[j] = __hip_atomic_fetch_min(g.depth + u[j], nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 #pragma unroll
-    for (int j = 0; j < kShortSplit; ++j) hits |= (old[j] > nd ? 1u : 0u) << j;
+    for (int j = 0; j < kC; ++j) hits |= (old[j] > nd ? 1u : 0u) << j;
     while (hits) {
         const int j = __builtin_ctz(hits);
         hits &= hits - 1u;
         int32_t v = u[0];
 #pragma unroll
-        for (int k = 1; k < kShortSplit; ++k) v = j == k ? u[k] : v;
+        for (int k = 1; k < kC; ++k) v = j == k ? u[k] : v;
         const int32_t us = g.row[v], ue = g.row[v + 1];
         if (us < 0 || ue < us || (int64_t)ue > g.ne)  // malformed offsets: never read past col
             GTAP_DEVICE_ERROR(*lane.dev, GTAP_ERROR_INVALID_ARGUMENT, lane.tid, -1, v, g.nv);
@@ -304,6 +330,8 @@ __device__ __forceinline__ void Program<NQ, kFlat>::run(L& lane) {
     const int32_t d = lane.template arg<int32_t>(12);
     // else v was reached by a shorter path meanwhile
     if (ld32(reinterpret_cast<const int32_t*>(g.depth) + v) >= d) {
+        if constexpr (kFlat) lane.coop_arg |= e - s > g.hub ? 1u : 0u;
+        const bool flat = kFlat && ballot(lane.coop_arg) != 0ull;
         if (e - s > g.split) {
             // up to kSplitFanout near-equal pieces, each routed by its own length
             const int64_t len = (int64_t)e - s;
@@ -315,7 +343,12 @@ __device__ __forceinline__ void Program<NQ, kFlat>::run(L& lane) {
                 __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
             }
         } else if constexpr (kFlat) {
-            lane.coop = true;  // its edges: run_coop
+            if (flat) {
+                lane.coop = true;  // its edges: run_coop
+            } else {
+                constexpr int32_t kC = kLaneEdges<NQ>;
+                for (int32_t at = s; at < e; at += kC) lane_scan<NQ>(lane, g, at, e - at < kC ? e : at + kC, d + 1);
+            }
         } else {
             lane_scan<NQ>(lane, g, s, e, d + 1);
         }
@@ -473,7 +506,13 @@ extern "C" int gtap_bfs(const int32_t* row, const int32_t* col, int32_t nv, int6
     bfs::BfsArg root{source, rs[0], rs[1], 0};
     const uint32_t q = (num_queues == 4) ? bfs::degree_bucket(rs[1] - rs[0]) : 0u;
     gtap_job job = host::make_job(bfs::F_BFS, q, &root, sizeof(root));
-    bfs::BfsArgs a{row, col, depth, nv, split, ne};
+    bfs::BfsArgs a{row, col, depth, nv, split, ne, -1};
+    // Large graphs may have no hubs (lane_scan): a range is one where degrees drawn at random around
+    // the mean would hardly ever reach.
+    const double mean = (double)ne / nv;
+    if (nv > (1 << 19) && (num_queues == 1 || mean >= 8.0)) {
+        a.hub = (int32_t)std::min(mean + 6.0 * std::sqrt(mean) + 8.0, 1e9);
+    }
     if (num_queues == 4) return host::run_single_job<Bfs4>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
     if (split <= bfs::kShortSplit) return host::run_single_job<Bfs1Short>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
     return host::run_single_job<Bfs1>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
@@ -500,7 +539,7 @@ extern "C" int gtap_bfs_block(const int32_t* row, const int32_t* col, int32_t nv
         return host::invalid_argument("gtap_bfs_block: bad source row offsets");
     bfs::BfsArg root{source, rs[0], rs[1], 0};
     gtap_job job = host::make_job(bfs::F_BFS, 0, &root, sizeof(root));
-    bfs::BfsArgs a{row, col, depth, nv, 0, ne};
+    bfs::BfsArgs a{row, col, depth, nv, 0, ne, 0};
     return host::run_single_block_job<bfs::BlockProgram>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);
 }
 

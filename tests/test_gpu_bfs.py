@@ -181,6 +181,24 @@ def test_bfs_flat_edge_windows(degrees, queues, split):
     assert np.array_equal(depth, oracle.bfs(row, col, 0))
 
 
+@pytest.mark.parametrize("queues,split", [(1, 64), (1, 17), (4, 64)])
+@pytest.mark.parametrize("nv,degree", [(1 << 19, 8), ((1 << 19) + 1, 8), (600_000, 3), (600_000, 9)])
+@pytest.mark.parametrize("hubs", [0, 1, 40])
+def test_bfs_large_graphs_with_and_without_hubs(queues, split, nv, degree, hubs):
+    """Graphs above 2^19 vertices are searched one range per lane until a wave meets a hub (ranges
+    of 7 to 15 edges here, hubs of 60 and 700): none, one deep in the graph, and several."""
+    print(f"case bfs large nv={nv} degree={degree} hubs={hubs} queues={queues} split={split}", flush=True)
+    rng = np.random.default_rng(nv + degree + hubs)
+    deg = rng.integers(degree - 2, degree + 3, nv)
+    at = rng.choice(np.arange(nv // 2, nv), hubs, replace=False)
+    deg[at] = np.where(np.arange(hubs) % 2 == 0, 700, 60)
+    row = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = rng.integers(0, nv, row[-1]).astype(np.int32)
+    depth, st = gtap_amd.bfs(row, col, 0, num_queues=queues, split=split)
+    assert st["error_code"] == 0
+    assert np.array_equal(depth, oracle.bfs(row, col, 0))
+
+
 @pytest.mark.parametrize("split", [1, 2, 15, 16, 17])
 @pytest.mark.parametrize("degrees", [[1] * 100, [15, 16, 17, 0, 1] * 30, [32, 33, 128, 129, 0, 1025] * 10])
 def test_bfs_short_splits(degrees, split):
