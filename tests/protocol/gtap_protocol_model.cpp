@@ -9,7 +9,9 @@
 //          kMargin of the top it last saw. Invariant: every task id is taken exactly once.
 //  ring    the id rings of 64-id cells with Vyukov sequence numbers (ring_put_claim,
 //          ring_probe / refill_chunk): producers take an enqueue ticket and wait for the cell,
-//          consumers CAS the dequeue position of a full cell. Invariant: every id once.
+//          consumers CAS the dequeue position of a full cell; the reset between launches gives
+//          up what is left and keeps the positions (drain_id_ring in gtap_host.hip). Invariant:
+//          every id once, from any position, over laps and the wrap of 32 bits.
 //  quiesce the all-tasks termination rule (thread_scheduler's idle path): idle count compared
 //          with the started count, job owners counted as started by the reset. Invariant:
 //          done is never set while a task is outstanding, also when the job owner starts
@@ -17,7 +19,7 @@
 //          they start) is shown to end early in that schedule. Also run with the idle count
 //          joined only after 4 consecutive failed acquire passes (kIdleRegisterAfter).
 //  ovf     the deque overflow rings (gtap_thread.hpp ovf_fill / ovf_pop / ovf_spill_deque,
-//          ovf_drain_kernel in gtap_host.hip): cells of state | position tag | id, a ticket
+//          drain_ovf_ring in gtap_host.hip): cells of state | position tag | id, a ticket
 //          fetch-add per batch, producers wait for the cell of the previous lap to be freed,
 //          consumers CAS the head over a run of READY cells and free them for the next lap;
 //          the drain frees what an aborted launch left between head and tickets. Invariant:
@@ -181,8 +183,24 @@ struct Ring {
     std::atomic<uint32_t> enq{0}, deq{0};
     std::vector<std::atomic<uint32_t>> seq;
     std::vector<std::atomic<uint32_t>> ids;
-    explicit Ring(uint32_t n) : ncells(n), seq(n), ids((size_t)n * kChunk) {
-        for (uint32_t i = 0; i < n; ++i) seq[i].store(i);
+    // Positions are never reset: `start` is where earlier launches have left them.
+    explicit Ring(uint32_t n, uint32_t start = 0) : ncells(n), seq(n), ids((size_t)n * kChunk) {
+        enq.store(start);
+        deq.store(start);
+        for (uint32_t i = 0; i < n; ++i) seq[(start + i) & (n - 1)].store(start + i);
+    }
+    // drain_id_ring of the reset kernel, with no launch running: the ids of full cells are given up
+    void drain() {
+        const uint32_t d = deq.load(), e = enq.load();
+        for (uint32_t i = 0; i < e - d; ++i) seq[(d + i) & (ncells - 1)].store(d + i + ncells);
+        deq.store(e);
+    }
+    // every cell free for its next lap
+    bool empty() const {
+        const uint32_t e = enq.load();
+        bool ok = deq.load() == e;
+        for (uint32_t i = 0; i < ncells; ++i) ok = ok && seq[(e + i) & (ncells - 1)].load() == e + i;
+        return ok;
     }
     void put(const uint32_t* v) {
         const uint32_t pos = enq.fetch_add(1, std::memory_order_relaxed);  // ticket
@@ -210,8 +228,15 @@ struct Ring {
     }
 };
 
-void run(unsigned seed, int producers, int consumers, uint32_t cells_each, uint32_t ncells) {
-    Ring ring(ncells);
+void run(unsigned seed, int producers, int consumers, uint32_t cells_each, uint32_t ncells, uint32_t start) {
+    Ring ring(ncells, start);
+    // what an earlier launch left: some cells full, given up by the reset
+    for (uint32_t k = 0, left = seed % ncells; k < left; ++k) {
+        const uint32_t v[kChunk] = {};
+        ring.put(v);
+    }
+    ring.drain();
+    CHECK(ring.empty(), "ring: a drain from position %u left cells", start);
     const uint32_t total = (uint32_t)producers * cells_each * kChunk;
     std::vector<std::atomic<uint8_t>> seen(total);
     for (auto& s : seen) s.store(0);
@@ -245,6 +270,7 @@ void run(unsigned seed, int producers, int consumers, uint32_t cells_each, uint3
     uint32_t missing = 0;
     for (uint32_t i = 0; i < total; ++i) missing += seen[i].load() == 0;
     CHECK(missing == 0, "ring: %u ids lost", missing);
+    CHECK(ring.empty(), "ring: emptied from position %u, cells not free", start);
 }
 
 }  // namespace ring_model
@@ -293,7 +319,7 @@ struct Ring {
         }
         return k;
     }
-    // ovf_drain_kernel, with no launch running
+    // drain_ovf_ring, with no launch running
     void drain() {
         const uint64_t h = head.load(), tk = tickets.load();
         for (uint64_t p = h; p < tk; ++p) cell(p).store(free_word(p + cap));
@@ -579,7 +605,8 @@ int main(int argc, char** argv) {
     const unsigned seeds = argc > 1 ? (unsigned)atoi(argv[1]) : 4;
     for (unsigned s = 1; s <= seeds; ++s) {
         deque_model::run(s, 3, 20000 + 1000 * s);
-        ring_model::run(s, 3, 3, 200, 64);
+        // from the start, from just below a lap's end, and over the wrap of the 32-bit positions
+        for (uint32_t start : {0u, 61u, 0xFFFFFFC0u - 3u, 0xFFFFFFFEu}) ring_model::run(s, 3, 3, 200, 64, start);
         join_model::run(s, 4095, s % 16, 4);
         join_model::run(s + 100, 1 + (int)(s * 37 % 4095), 15, 3);
         const bool early = quiesce_model::run(s, 6, 1, 2000, true, 0);

@@ -55,9 +55,9 @@ def test_admission_holds_jobs_back_and_results_stay_exact():
 
 def test_id_rings_carry_over_launches():
     """The id rings keep their positions from launch to launch; what a launch leaves in them is
-    given up by the next one's reset. Served runs on a small pool park few ids per wave and so
-    pass ids through the rings; their leftovers must not be handed out again in later launches
-    (a doubled id would break results), and a launch that ends in an error must not either."""
+    given up by the next one's reset. Served, fork-join, block-mode and failing launches in turn on
+    one pool stay exact (a doubled id would break results); the rings' own state is read back in
+    test_gpu_overflow_star.py."""
     st = gtap_amd.Stream(seed=47, njobs=200)
     try:
         exp = expected(st)
