@@ -20,7 +20,7 @@
 //           int u = col[i];
 //           if (atomicMin(&depth[u], d + 1) > d + 1) {
 //               #pragma gtap task queue(bucket(row[u + 1] - row[u]))
-//               bfs(u, row[u], row[u + 1], d + 1);   // (not for a u without out-edges)
+//               bfs(u, row[u], row[u + 1], d + 1);   // (the flat scan: not for a u without out-edges)
 //           }
 //       }
 //   }

@@ -262,8 +262,9 @@ using SpmvProgram = gtap::spmv::Program;
 static_assert(SpmvProgram::kFrameBytes + gtap::kHdrBytes <= gtap::host::kBuiltinStride, "frame exceeds stride");
 
 // y = A x for a CSR matrix already in device memory (row_ptr: rows+1 int32, col_idx: nnz
-// int32, val: nnz float64, x: cols float64, y: rows float64). Rows are split in halves down to
-// ranges of at most `cutoff` rows (0 -> 16), whose rows become one task each.
+// int32, val: nnz float64, x: cols float64, y: rows float64). Rows are split in 4 pieces (in 2
+// where full batches of `cutoff` rows do not fit the deque) down to ranges of at most `cutoff` rows
+// (0 -> 16), whose rows become one task each.
 // Replaces the program of examples/spmv/spmv_thread.cu:34-66.
 extern "C" int gtap_spmv(const int32_t* row_ptr, const int32_t* col_idx, const double* val, const double* x,
                          double* y, int32_t rows, int32_t cols, int32_t cutoff, gtap_run_stats* stats) {
