@@ -69,6 +69,9 @@ __host__ __device__ __forceinline__ uint32_t degree_bucket(int32_t deg) {
     return deg < 8 ? 0u : (deg < 64 ? 1u : (deg < 512 ? 2u : 3u));
 }
 
+// Set in the depth of a piece of a hub's range (depths are at most 0x3f3f3f3f), so that the wave that
+// takes the piece knows too.
+constexpr int32_t kHubPiece = 1 << 30;
 constexpr int32_t kSplitFanout = 8;         // pieces per split of a lane task's range
 constexpr int32_t kWaveSplitEdges = 2048;  // a wave task scans at most this many edges (and cap / 8)
 constexpr int kWindows = 8;                 // edges per lane per step of an expansion
@@ -275,10 +278,11 @@ __device__ __forceinline__ void expand(T& t, const BfsArgs& g, ExpandShared* sh,
 //   search expands more vertices twice. Uniform random graphs of 4M vertices and 4 / 8 / 16 edges a
 //   vertex, flat with batches of 32 / per lane (us): one queue 2350 / 1455, 3180 / 1910, 3610 / 2440;
 //   four queues (batches of 64) 1548 / 1438, 2200 / 1830, 3600 / 2430; 1M vertices of 16 edges 484 /
-//   473 and 648 / 487. A graph is large here above 2^19 vertices (400K vertices with 16 edges a
-//   vertex, their ends drawn at random: flat 325, per lane 384 us) and, with four queues, of at
-//   least 8 edges a vertex (1M vertices of 4 drawn edges: 546 / 700 us). R-MAT graphs have hubs:
-//   their waves turn to the flat scan within a round or two and keep its gain.
+//   473 and 648 / 487. A graph is large here above 3 * 2^18 vertices with one queue (700K vertices
+//   with 6 or 16 edges a vertex, their ends drawn at random: 342 / 375 and 419 / 433 us; 1M with
+//   4: 409 / 397), above 2^19 with four (700K, 16: 530 / 483 us; 524K, 16: the same) and there of at
+//   least 8 edges a vertex (1M, 4: 546 / 700 us). R-MAT graphs have hubs: their waves turn to the flat
+//   scan within a round or two and keep its gain.
 constexpr int32_t kShortSplit = 16;
 template <int NQ>
 constexpr int32_t kLaneEdges = NQ == 4 ? 8 : kShortSplit;  // with four queues 16 spill 20 registers, 8 spill 7
@@ -327,20 +331,22 @@ __device__ __forceinline__ void Program<NQ, kFlat>::run(L& lane) {
     const int32_t v = lane.template arg<int32_t>(0);
     const int32_t s = lane.template arg<int32_t>(4);
     const int32_t e = lane.template arg<int32_t>(8);
-    const int32_t d = lane.template arg<int32_t>(12);
+    const int32_t piece = lane.template arg<int32_t>(12) & kHubPiece;
+    const int32_t d = lane.template arg<int32_t>(12) & ~kHubPiece;
     // else v was reached by a shorter path meanwhile
     if (ld32(reinterpret_cast<const int32_t*>(g.depth) + v) >= d) {
-        if constexpr (kFlat) lane.coop_arg |= e - s > g.hub ? 1u : 0u;
+        if constexpr (kFlat) lane.coop_arg |= piece != 0 || e - s > g.hub ? 1u : 0u;
         const bool flat = kFlat && ballot(lane.coop_arg) != 0ull;
         if (e - s > g.split) {
             // up to kSplitFanout near-equal pieces, each routed by its own length
             const int64_t len = (int64_t)e - s;
             int32_t k = (int32_t)((len + g.split - 1) / g.split);
             if (k > kSplitFanout) k = kSplitFanout;
+            const int32_t pd = d | (kFlat && (piece != 0 || e - s > g.hub) ? kHubPiece : 0);
             for (int32_t i = 0; i < k; ++i) {
                 const int32_t ps = s + (int32_t)(len * i / k);
                 const int32_t pe = s + (int32_t)(len * (i + 1) / k);
-                __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
+                __gtap_spawn_task_detached(lane, F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, pd});
             }
         } else if constexpr (kFlat) {
             if (flat) {
@@ -360,7 +366,7 @@ template <int NQ, bool kFlat>
 template <class L>
 __device__ __forceinline__ void Program<NQ, kFlat>::run_coop(L& lane, uint64_t mask, WaveShared* sh) {
     (void)mask;
-    const int32_t s = (int32_t)lane.frame[1], nd = (int32_t)lane.frame[3] + 1;
+    const int32_t s = (int32_t)lane.frame[1], nd = ((int32_t)lane.frame[3] & ~kHubPiece) + 1;
     int32_t left = lane.coop ? (int32_t)lane.frame[2] - s : 0, at = s;
     do {
         const int32_t n = left < kMaxExpand ? left : kMaxExpand;
@@ -378,7 +384,7 @@ __device__ __forceinline__ void Program<NQ, kFlat>::run_wave(W& wt) {
     const int32_t v = wt.template arg<int32_t>(0);
     const int32_t s = wt.template arg<int32_t>(4);
     const int32_t e = wt.template arg<int32_t>(8);
-    const int32_t d = wt.template arg<int32_t>(12);
+    const int32_t d = wt.template arg<int32_t>(12) & ~kHubPiece;
     if (wt.func != F_BFS) {
         if (wt.lane == 0) GTAP_DEVICE_ERROR(*wt.dev, GTAP_ERROR_INVALID_FUNCTION, wt.tid, wt.queue, wt.func, F_BFS);
         wt.finish();
@@ -400,7 +406,7 @@ __device__ __forceinline__ void Program<NQ, kFlat>::run_wave(W& wt) {
         if (wt.lane < k) {
             const int32_t ps = s + (int32_t)(len * wt.lane / k);
             const int32_t pe = s + (int32_t)(len * (wt.lane + 1) / k);
-            wt.spawn_detached_lane(F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d});
+            wt.spawn_detached_lane(F_BFS, route<NQ>(pe - ps), BfsArg{v, ps, pe, d | kHubPiece});
         }
         wt.finish();
         return;
@@ -510,7 +516,7 @@ extern "C" int gtap_bfs(const int32_t* row, const int32_t* col, int32_t nv, int6
     // Large graphs may have no hubs (lane_scan): a range is one where degrees drawn at random around
     // the mean would hardly ever reach.
     const double mean = (double)ne / nv;
-    if (nv > (1 << 19) && (num_queues == 1 || mean >= 8.0)) {
+    if (nv > (num_queues == 1 ? 3 << 18 : 1 << 19) && (num_queues == 1 || mean >= 8.0)) {
         a.hub = (int32_t)std::min(mean + 6.0 * std::sqrt(mean) + 8.0, 1e9);
     }
     if (num_queues == 4) return host::run_single_job<Bfs4>(a, job, nullptr, stats, GTAP_TERM_QUIESCE);

@@ -182,11 +182,12 @@ def test_bfs_flat_edge_windows(degrees, queues, split):
 
 
 @pytest.mark.parametrize("queues,split", [(1, 64), (1, 17), (4, 64)])
-@pytest.mark.parametrize("nv,degree", [(1 << 19, 8), ((1 << 19) + 1, 8), (600_000, 3), (600_000, 9)])
+@pytest.mark.parametrize("nv,degree", [(1 << 19, 8), ((1 << 19) + 1, 8), (3 << 18, 3), ((3 << 18) + 1, 3), (800_000, 9)])
 @pytest.mark.parametrize("hubs", [0, 1, 40])
 def test_bfs_large_graphs_with_and_without_hubs(queues, split, nv, degree, hubs):
-    """Graphs above 2^19 vertices are searched one range per lane until a wave meets a hub (ranges
-    of 7 to 15 edges here, hubs of 60 and 700): none, one deep in the graph, and several."""
+    """Large graphs (above 3 * 2^18 vertices with one queue, 2^19 with four) are searched one range per
+    lane until a wave meets a hub or a piece of one (ranges of 1 to 11 edges here, hubs of 60 and 700,
+    which splits of 64 and 17 cut): none, one deep in the graph, and several."""
     print(f"case bfs large nv={nv} degree={degree} hubs={hubs} queues={queues} split={split}", flush=True)
     rng = np.random.default_rng(nv + degree + hubs)
     deg = rng.integers(degree - 2, degree + 3, nv)
